@@ -298,7 +298,8 @@ struct Params {
   // Launch shape (packed kernels): grid workgroups (0: tiles_m * tiles_n).
   // A K-split launch (ksplit s > 1, grid s u) gives workgroup h u + w the
   // tile tile_base + w and share h of its S K stages, stages
-  // floor(h S / s) .. floor((h + 1) S / s) - 1 (S >= s), and stores that
+  // floor(h S / s) .. floor((h + 1) S / s) - 1 (S >= s; the cubic divides its
+  // S / 2 pairs of stages so, see work_share), and stores that
   // share as a dense FP32 block (dense_share_output): share h of split tile
   // w at h * split_stride + w * kSplitTileFloats floats, split_stride =
   // u * kSplitTileFloats.
@@ -319,6 +320,9 @@ struct WorkShare {
   int share;    // 0 .. ksplit-1
 };
 
+// kUnit: stages that stay together. The cubic's main loop takes two stages
+// per turn, so an odd share of it would add its last stage twice.
+template <int kUnit>
 __device__ __forceinline__ WorkShare work_share(const Params& p, int nstages_all) {
   WorkShare w;
   if (p.ksplit > 1) {
@@ -329,8 +333,9 @@ __device__ __forceinline__ WorkShare work_share(const Params& p, int nstages_all
     const uint32_t share = blockIdx.x / tiles;
     w.share = (int)share;
     w.tile = p.tile_base + (int)(blockIdx.x - share * tiles);
-    w.stage0 = (int)(share * (uint32_t)nstages_all / (uint32_t)p.ksplit);
-    w.nstages = (int)((share + 1) * (uint32_t)nstages_all / (uint32_t)p.ksplit) - w.stage0;
+    const uint32_t units = (uint32_t)nstages_all / kUnit;
+    w.stage0 = kUnit * (int)(share * units / (uint32_t)p.ksplit);
+    w.nstages = kUnit * (int)((share + 1) * units / (uint32_t)p.ksplit) - w.stage0;
     // The divisions run on VALU; the results are uniform, and in SGPRs they
     // leave the VGPRs to the accumulators.
     w.share = __builtin_amdgcn_readfirstlane(w.share);

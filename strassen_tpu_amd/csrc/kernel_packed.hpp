@@ -152,7 +152,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_packed(Params p) {
   const int wm = wave >> 1, wn = wave & 1;
 
   const int nstages_all = (int)(p.k / (2 * TK));
-  const WorkShare ws = work_share(p, nstages_all);
+  const WorkShare ws = work_share<2>(p, nstages_all);
   int tile_m, tile_n;
   tile_of(ws.tile, p.tiles_m, p.tiles_n, p.group_m, p.raster, tile_m, tile_n);
   TileOrigin o = tile_origin<kThin>(p, (int64_t)tile_m * TM, (int64_t)tile_n * TN);

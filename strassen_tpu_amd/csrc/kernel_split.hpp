@@ -386,7 +386,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_split(Params p) {
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int nstages_all = (int)(p.k / (2 * TK));
-  const WorkShare ws = work_share(p, nstages_all);
+  const WorkShare ws = work_share<1>(p, nstages_all);
   int tile_m, tile_n;
   tile_of(ws.tile, p.tiles_m, p.tiles_n, p.group_m, p.raster, tile_m, tile_n);
   // The tile indices are uniform, but the integer divisions that produce

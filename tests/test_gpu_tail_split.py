@@ -399,3 +399,21 @@ def test_small_thin_launch_qk_norm_rope(algo):
     want = _oracle(algo, x, laid, tile, epilogue="qk_norm_rope", rope_cos=tcos, rope_sin=tsin, rope_scale=scale,
                    rope_head_dim=128, rope_eps=1e-6)
     assert_ulp_close(got, want, k=k)
+
+
+@pytest.mark.parametrize("algo", [7, 8])
+@pytest.mark.parametrize("shape,tile", [((256, 8704, 512), (256, 256, 512)), ((48, 8192, 5120), (16, 256, 512))])
+def test_shares_that_do_not_divide_the_stages(algo, shape, tile):
+    """Share counts that leave an odd number of stages per share when K's
+    stages are divided evenly (272 stages in 16 shares, 256 in 12): integer
+    operands come out bit-exact, so no stage is missed or added twice."""
+    (m, k, n), bm = shape, tile[0]
+    _, split, s = _plan(m, n, k, bm)
+    if not split or all(((h + 1) * (k // 32) // s - h * (k // 32) // s) % 2 == 0 for h in range(s)):
+        pytest.skip("this device's CU count splits this shape evenly, or SMX_TAIL_SPLIT=0")
+    rng = np.random.default_rng(5 + algo)
+    a = rng.integers(-2, 3, (m, k)).astype(np.float32)
+    b = rng.integers(-2, 3, (k, n)).astype(np.float32)
+    pa, pb = _pack(algo, a, b, tile)
+    got, _ = abi_gemm(algo, pa, pb, m, n, k, tile, workspace=True, out_f32=True)
+    assert np.array_equal(host(got), a @ b)

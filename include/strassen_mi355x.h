@@ -41,7 +41,7 @@
 extern "C" {
 #endif
 
-#define SMX_VERSION 12
+#define SMX_VERSION 13
 
 /* Status codes. */
 #define SMX_OK 0
@@ -226,6 +226,28 @@ int smx_gemm_noalloc(const smx_gemm_desc* desc, const void* a, const void* b, vo
  * the reference (a launch shape of gfx950). A row-major A with a packed B
  * (smx_gemm_noalloc's descriptor) is sized as the packed call it becomes. */
 int smx_gemm_workspace_bytes(const smx_gemm_desc* desc, int64_t* bytes);
+
+/*
+ * One matrix product on a packed weight, the library choosing how it runs.
+ * Takes smx_gemm's descriptor with b_layout = SMX_B_PACKED and A either
+ * packed (a_layout = SMX_A_PACKED) or row-major [m, k / passes] (row stride
+ * lda, rows 16-byte aligned; a_dtype SMX_DTYPE_BF16, or SMX_DTYPE_F32 with
+ * passes 1, 3 or 6 as for smx_pack_operand: desc->k is the packed K), which
+ * the call packs into the workspace first. Launches with few product rows or
+ * few tiles (decode-sized M, small squares) then run on the streaming
+ * kernel, whose tiles are smaller and which takes operands straight from
+ * memory to registers; other calls run as smx_gemm runs them (flags choose
+ * the Strassen kernel; a Strassen call without
+ * SMX_FLAG_PRODUCT_MAJOR_ROUNDS never takes the streaming kernel). Results
+ * match smx_gemm's up to the order of FP32 additions. desc->workspace must
+ * hold smx_matmul_workspace_bytes(desc, ...) bytes (16-byte aligned; NULL
+ * when that is 0); every argument is checked before anything is launched.
+ * No counterpart in the reference (kernel choice of gfx950).
+ */
+int smx_matmul(const smx_gemm_desc* desc, int32_t a_dtype, int32_t passes, const void* a, const void* b, void* c,
+               const void* residual, const void* bias, const void* rope_cos, const void* rope_sin,
+               const void* rope_scale, void* stream);
+int smx_matmul_workspace_bytes(const smx_gemm_desc* desc, int32_t a_dtype, int32_t passes, int64_t* bytes);
 
 /* Tile granules of the kernels that serve (algo, epilogue, b_layout): bm
  * must be a multiple of 2*tm, bn of 2*tn, bk of 2*tk. Packed operands: 8, 128,

@@ -58,8 +58,8 @@ SMX_NRA_OUT_F32 = 4
 SMX_QK_SCALE_F32 = 1
 SMX_QK_OUT_F32 = 4
 
-EXPORTS = ("smx_gemm", "smx_gemm_noalloc", "smx_gemm_workspace_bytes", "smx_tile_requirements", "smx_packed_bytes", "smx_pack_operand",
-           "smx_norm_residual_add", "smx_qk_norm_rope", "smx_last_error", "smx_version")
+EXPORTS = ("smx_gemm", "smx_gemm_noalloc", "smx_gemm_workspace_bytes", "smx_matmul", "smx_matmul_workspace_bytes",
+           "smx_tile_requirements", "smx_packed_bytes", "smx_pack_operand", "smx_norm_residual_add", "smx_qk_norm_rope", "smx_last_error", "smx_version")
 
 
 class SmxGemmDesc(ctypes.Structure):
@@ -105,6 +105,10 @@ def load():
                                           ctypes.POINTER(ctypes.c_int32)]
     lib.smx_tile_requirements.restype = ctypes.c_int
     i64, i32 = ctypes.c_int64, ctypes.c_int32
+    lib.smx_matmul.argtypes = [ctypes.POINTER(SmxGemmDesc), i32, i32, vp, vp, vp, vp, vp, vp, vp, vp, vp]
+    lib.smx_matmul.restype = ctypes.c_int
+    lib.smx_matmul_workspace_bytes.argtypes = [ctypes.POINTER(SmxGemmDesc), i32, i32, ctypes.POINTER(i64)]
+    lib.smx_matmul_workspace_bytes.restype = ctypes.c_int
     lib.smx_packed_bytes.argtypes = [i32, i64, i64, ctypes.POINTER(i64)]
     lib.smx_packed_bytes.restype = ctypes.c_int
     lib.smx_pack_operand.argtypes = [i32, i32, i32, i32, i64, i64, vp, i32, i32, i64, i32, i32, vp, i64, vp, vp]

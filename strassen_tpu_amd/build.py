@@ -1,7 +1,7 @@
 """Build the gfx950 C-ABI library in-tree.
 
 ``python -m strassen_tpu_amd.build`` (or ``build()``) compiles the C ABI's
-translation unit (``csrc/strassen_gemm.hip``) and the four units that
+translation unit (``csrc/strassen_gemm.hip``) and the six units that
 instantiate the GEMM kernels (``csrc/gemm_*.hip``) with hipcc, in parallel,
 checks each unit's device assembly, and links ``libstrassen_mi355x.so`` next
 to this file. hipcc cross-compiles for gfx950 without a GPU.
@@ -21,7 +21,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 REPO = os.path.dirname(HERE)
 SOURCES = tuple(os.path.join(HERE, "csrc", name) for name in (
     "strassen_gemm.hip", "gemm_strassen.hip", "gemm_strassen_thin.hip", "gemm_strassen_pm.hip", "gemm_cubic.hip",
-    "gemm_cubic_thin.hip"))
+    "gemm_cubic_thin.hip", "gemm_stream.hip"))
 LIBRARY = os.path.join(HERE, "libstrassen_mi355x.so")
 INCLUDE = os.path.join(REPO, "include")
 
@@ -124,6 +124,7 @@ def verify_inline_asm_kernels(asm_text):
 _KERNEL_DESC = re.compile(r"\.amdhsa_kernel (\S+)(.*?)\.end_amdhsa_kernel", re.S)
 _SPLIT = re.compile(r"gemm_splitILi(\d+)ELi(\d+)ELb(\d)E")
 _PM = re.compile(r"gemm_pmILi(\d+)EE")
+_STREAM = re.compile(r"gemm_streamILi(\d+)E")
 _PACKED = re.compile(r"gemm_packedILi(\d+)ELi(\d+)ELi(\d+)ELi(\d+)ELb(\d)E")
 _QUAD_CUBIC_PARTIAL = 1
 PARTIAL_SCRATCH_CAP = 1024
@@ -131,7 +132,7 @@ PARTIAL_SCRATCH_CAP = 1024
 
 def scratch_limit(name):
     """Allowed scratch bytes per lane of a kernel (None: not a GEMM kernel)."""
-    if _SPLIT.search(name) or _PM.search(name):
+    if _SPLIT.search(name) or _PM.search(name) or _STREAM.search(name):
         return 0
     m = _PACKED.search(name)
     if m:
@@ -189,10 +190,12 @@ def build(verbose=False, jobs=None):
             if verbose and stderr.strip():
                 print(stderr, file=sys.stderr)
             # The C ABI's unit holds the compact kernels and the packers; the
-            # inline-asm MFMA kernels and the GEMM scratch limits live in the
-            # kernel units, each of which must hold some.
-            kernel_unit = os.path.basename(source) != "strassen_gemm.hip"
-            if kernel_unit:
+            # GEMM scratch limits live in the kernel units, each of which must
+            # hold some, and inline-asm MFMAs in all of those but the streaming
+            # kernels', whose MFMAs are the compiler's builtins.
+            unit = os.path.basename(source)
+            kernel_unit = unit != "strassen_gemm.hip"
+            if kernel_unit and unit != "gemm_stream.hip":
                 checked += verify_inline_asm_kernels(text)
             gemms += verify_kernel_scratch(text, require=kernel_unit)
         cmd = link_command([obj for obj, _, _ in units], tmp)

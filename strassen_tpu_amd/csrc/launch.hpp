@@ -40,6 +40,25 @@ int launch_cubic(const Params& p, int epilogue, hipStream_t stream);
 // 128 x 256 product-space tiles, p.tiles_n counted in those, p.park set.
 int launch_strassen_pm(const Params& p, int epilogue, hipStream_t stream);
 
+// Tilings of the streaming kernel (kernel_stream.hpp): 32 rb x 32 cb of
+// product space per workgroup, for launches of one tile row (whose B loads
+// stream past the L2) or of several.
+struct StreamShape {
+  int algo, rb, cb;
+  bool one_row;
+};
+constexpr StreamShape kStreamShape[] = {
+    {7, 1, 2, true}, {7, 1, 4, true}, {7, 2, 2, true}, {7, 2, 4, true}, {7, 1, 1, false},
+    {7, 2, 2, false}, {8, 1, 2, true}, {8, 1, 4, true}, {8, 2, 2, true}, {8, 1, 1, false}, {8, 2, 2, false},
+};
+constexpr int kStreamShapes = sizeof(kStreamShape) / sizeof(kStreamShape[0]);
+
+// The streaming kernel in tiling kStreamShape[shape] on packed operands
+// (p.tiles_m x p.tiles_n of its tiles, p.ksplit shares of K, p.epilogue).
+// With several shares p.park takes them and launch_stream_sum follows.
+int launch_stream(const Params& p, int shape, hipStream_t stream);
+int launch_stream_sum(const Params& p, hipStream_t stream);
+
 extern template int launch_strassen<false>(const Params&, int, hipStream_t);
 extern template int launch_strassen<true>(const Params&, int, hipStream_t);
 extern template int launch_cubic<false>(const Params&, int, hipStream_t);

@@ -31,6 +31,9 @@
 //      tiles, 64x64 waves, both operands pre-packed (smx_pack_operand: the
 //      Strassen operand sums or the cubic quadrants, in MFMA fragment order)
 //      and streamed into an LDS ring by DMA.
+//   stream (kernel_stream.hpp): launches of few product rows or few tiles
+//      (smx_matmul): tiles of 32 to 128 rows and columns, one product per wave,
+//      operands straight from memory into registers.
 //   v1 (kernel_v1.hpp): 128x64 tiles, row-major A and B^T, both operand sums
 //      formed in registers; serves unpacked calls whose tile the packed
 //      kernels cannot take, or all of them under SMX_PLAIN_WEIGHTS=compact.
@@ -696,6 +699,107 @@ int launch_rest(Params p, const smx_gemm_desc& d, hipStream_t s) {
   return launch_split_fixup(f, d.epilogue, (const float*)d.workspace, plan.split, s);
 }
 
+// How smx_matmul runs a packed call on the streaming kernel (kernel_stream.hpp):
+// one of its tilings and the shares of K. shape < 0: not at all.
+struct StreamPlan {
+  int shape = -1, shares = 1;
+};
+
+// Estimated time in us of a packed call on the 128 x 128 tile kernels (with
+// the K split that split_plan gives it): per tile and round 0.027 us of K
+// (Strassen) or 0.022 (cubic), three quarters of that while at most half the
+// CUs work, and 10 us around it; the packed weight at 4.4 TB/s; 8 us and the
+// shares' traffic for a split's second pass. Measured on MI355X, packed
+// operands: Strassen 16 x 512 x 1024 19 us (estimate 20), 1024^3 27 (31), 2048^3 48
+// (49), 16 x 5120 x 5120 37 (39), 256 x 25600 x 5120 128 (138), 256 x 5120 x
+// 51200 210 (218).
+double tile_kernel_us(const Params& p, int algo, int cus, const SplitPlan& plan, double packed_b) {
+  const int tiles = plan.whole + plan.split;
+  const double per_k = algo == SMX_ALGO_STRASSEN ? 0.027 : 0.022;
+  auto round_us = [&](int wgs, double k) { return k * per_k * (2 * wgs <= cus ? 0.75 : 1.0) + 10.0; };
+  double us = 0;
+  if (plan.split) {
+    const int wgs = plan.ksplit * plan.split;
+    us = (plan.whole / cus) * round_us(cus, (double)p.k) +
+         ((wgs + cus - 1) / cus) * round_us(wgs, (double)p.k / plan.ksplit) + 8.0 +
+         (double)plan.ksplit * plan.split * kSplitTileFloats * 8 / 8e6;
+    return std::max(us, packed_b / 4.4e6 + 18.0);
+  }
+  us = ((tiles + cus - 1) / cus) * round_us(tiles, (double)p.k);
+  return std::max(us, packed_b / 4.4e6 + 10.0);
+}
+
+// The streaming kernel's plan for a packed call, if it is expected to beat the
+// 128 x 128 tile kernels by a tenth. A workgroup of the streaming kernel
+// takes its operands at about 57 bytes a ns (70 where several tile rows
+// share B through the L2), the launch its weight at 6.4 TB/s (5.1 in more
+// than one round of workgroups, 4 where B is read by several tile rows), with
+// 3 us around it and, for a divided K, 4 us
+// and the FP32 shares' traffic for the summing launch. Measured, as above:
+// 16 x 512 x 1024 9 us (estimate 9), 1024^3 8 (9), 2048^3 28 (29), 16 x 5120 x 5120 21
+// (22), 64 x 25600 x 5120 77 (84), 16 x 5120 x 51200 141 (146). K is divided
+// until the workgroups fill the CUs once; every share keeps
+// kStreamMinStages stages.
+constexpr int kStreamMinStages = 8;
+
+int stream_plan(const Params& p, const smx_gemm_desc& d, StreamPlan* plan) {
+  *plan = StreamPlan{};
+  if (p.partial || (d.algo == SMX_ALGO_STRASSEN && !(d.flags & SMX_FLAG_PRODUCT_MAJOR_ROUNDS))) return SMX_OK;
+  int cus = 0;
+  if (int rc = device_cus(&cus)) return rc;
+  const int64_t prows = p.m / 2, stages = p.k / 32;
+  const double nops = packed::nops_of(d.algo);
+  const double packed_b = (double)p.n / 2 * (double)p.k / 2 * nops * 2;
+  Params q = p;
+  packed_grid(q, d.algo);
+  const int64_t whole_tiles = (int64_t)q.tiles_m * q.tiles_n;
+  if (whole_tiles > cus) return SMX_OK;  // over one round of tiles
+  SplitPlan split{};
+  if (int rc = split_plan(q, &split)) return rc;
+  double best = 0.9 * tile_kernel_us(q, d.algo, cus, split, packed_b);
+  for (int i = 0; i < kStreamShapes; ++i) {
+    const StreamShape& t = kStreamShape[i];
+    if (t.algo != d.algo) continue;
+    const int64_t rows = (prows + 32 * t.rb - 1) / (32 * t.rb);
+    if ((rows == 1) != t.one_row || (t.one_row && t.rb > 1 && prows <= 16 * t.rb)) continue;
+    // several tile rows re-read B: only where most CUs would idle
+    if (rows > 1 && whole_tiles > cus / 4) continue;
+    if (d.epilogue == SMX_EPI_QK_NORM_ROPE && t.cb < 2) continue;  // a head is 64 columns of a half
+    const int64_t tiles = rows * (p.n / (64 * t.cb));
+    const int64_t shares = std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(cus / tiles, kMaxKSplit),
+                                                                  stages / kStreamMinStages));
+    const int64_t rounds = (tiles * shares + cus - 1) / cus;
+    const double kb_per_stage = t.algo == SMX_ALGO_STRASSEN ? 7.0 * (t.rb + t.cb) : 4.0 * (2 * t.rb + t.cb);
+    const double wg_us = (double)rounds * ((stages + shares - 1) / shares) * kb_per_stage * 1.024 / (rows > 1 ? 70 : 57);
+    // a second, partly filled round of one-row workgroups leaves CUs idle at its end
+    double us = 3.0 + std::max(wg_us, packed_b / (rows > 1 ? 4e6 : rounds > 1 ? 5.1e6 : 6.4e6));
+    if (shares > 1) us += 4.0 + (double)shares * p.m * p.n * 8 / 8e6;
+    if (us < best) {
+      best = us;
+      plan->shape = i;
+      plan->shares = (int)shares;
+    }
+  }
+  return SMX_OK;
+}
+
+int64_t stream_bytes(const Params& p, const StreamPlan& plan) {
+  return plan.shares > 1 ? (int64_t)plan.shares * p.m * p.n * (int64_t)sizeof(float) : 0;
+}
+
+int launch_stream_plan(Params p, const smx_gemm_desc& d, const StreamPlan& plan, void* workspace, hipStream_t s) {
+  const StreamShape& t = kStreamShape[plan.shape];
+  p.tiles_m = (int)((p.m / 2 + 32 * t.rb - 1) / (32 * t.rb));
+  p.tiles_n = (int)(p.n / (64 * t.cb));
+  p.group_m = group_m_setting();
+  p.ksplit = plan.shares;
+  p.park = workspace;
+  p.split_stride = p.m * p.n;
+  p.epilogue = d.epilogue;
+  if (int rc = launch_stream(p, plan.shape, s)) return rc;
+  return plan.shares > 1 ? launch_stream_sum(p, s) : SMX_OK;
+}
+
 // Device scratch of smx_gemm_noalloc: the packed activation of one call,
 // at most kNoAllocScratchBytes. Each GPU the library runs on holds its own
 // copy from module load until the process ends. Host code never passes the
@@ -926,6 +1030,96 @@ int smx_gemm_noalloc(const smx_gemm_desc* d, const void* a, const void* b, void*
     return rc;
   p.a = (const uint16_t*)scratch_ptr;
   return launch_gemm(p, packed, (hipStream_t)stream);
+}
+
+}  // extern "C"
+
+namespace {
+
+// A smx_matmul call: the checked parameters of the packed call it becomes,
+// the space its packed A takes at the head of the workspace, and the
+// workspace of its GEMM behind that.
+struct MatmulCall {
+  smx_gemm_desc desc;
+  Params p{};
+  StreamPlan stream;
+  int64_t a_bytes = 0, gemm_bytes = 0;
+};
+
+int matmul_call(const smx_gemm_desc* d, int32_t a_dtype, int32_t passes, const void* b, void* c, const void* residual,
+                const void* bias, const void* rope_cos, const void* rope_sin, const void* rope_scale,
+                MatmulCall* call) {
+  if (!d) return fail(SMX_ERR_INVALID, "null descriptor");
+  if (d->b_layout != SMX_B_PACKED) return fail(SMX_ERR_UNSUPPORTED, "smx_matmul takes a packed B (SMX_B_PACKED)");
+  if (d->a_layout != SMX_A_ROWMAJOR && d->a_layout != SMX_A_PACKED)
+    return fail(SMX_ERR_INVALID, "a_layout must be SMX_A_ROWMAJOR or SMX_A_PACKED, got %d", d->a_layout);
+  if (a_dtype != SMX_DTYPE_BF16 && a_dtype != SMX_DTYPE_F32)
+    return fail(SMX_ERR_INVALID, "a_dtype must be SMX_DTYPE_BF16 (0) or SMX_DTYPE_F32 (1), got %d", a_dtype);
+  if (passes != 1 && passes != 3 && passes != 6)
+    return fail(SMX_ERR_INVALID, "passes must be 1, 3 or 6, got %d", passes);
+  MatmulCall& t = *call;
+  t.desc = *d;
+  t.desc.a_layout = SMX_A_PACKED;
+  t.desc.workspace = nullptr;
+  t.desc.workspace_bytes = 0;
+  if (int rc = gemm_params(&t.desc, kNoAllocScratchProbe, b, c, residual, bias, rope_cos, rope_sin, rope_scale, t.p))
+    return rc;
+  if (d->a_layout == SMX_A_ROWMAJOR) {
+    const int64_t bytes = packed::padded_product_rows(d->m) * (d->k / 2) * packed::nops_of(d->algo) * 2;
+    t.a_bytes = (bytes + 255) / 256 * 256;
+  }
+  if (int rc = stream_plan(t.p, t.desc, &t.stream)) return rc;
+  if (t.stream.shape >= 0) {
+    t.gemm_bytes = stream_bytes(t.p, t.stream);
+    return SMX_OK;
+  }
+  Parts parts;
+  if (int rc = plan_parts(t.p, t.desc, &parts)) return rc;
+  return parts_workspace(parts, &t.gemm_bytes);
+}
+
+}  // namespace
+
+extern "C" {
+
+int smx_matmul_workspace_bytes(const smx_gemm_desc* d, int32_t a_dtype, int32_t passes, int64_t* bytes) {
+  g_error[0] = 0;
+  if (!bytes) return fail(SMX_ERR_INVALID, "null output");
+  *bytes = 0;
+  const void* x = kNoAllocScratchProbe;
+  MatmulCall call;
+  if (int rc = matmul_call(d, a_dtype, passes, x, const_cast<void*>(x), x, x, x, x, x, &call)) return rc;
+  *bytes = call.a_bytes + call.gemm_bytes;
+  return SMX_OK;
+}
+
+int smx_matmul(const smx_gemm_desc* d, int32_t a_dtype, int32_t passes, const void* a, const void* b, void* c,
+               const void* residual, const void* bias, const void* rope_cos, const void* rope_sin,
+               const void* rope_scale, void* stream) {
+  g_error[0] = 0;
+  MatmulCall call;
+  if (int rc = matmul_call(d, a_dtype, passes, b, c, residual, bias, rope_cos, rope_sin, rope_scale, &call)) return rc;
+  if (!a) return fail(SMX_ERR_INVALID, "null operand pointer");
+  const int64_t need = call.a_bytes + call.gemm_bytes;
+  if (need && (!d->workspace || !aligned16(d->workspace) || d->workspace_bytes < need))
+    return fail(SMX_ERR_INVALID, "smx_matmul needs a 16-byte aligned workspace of %lld bytes "
+                "(smx_matmul_workspace_bytes), got %lld", (long long)need,
+                (long long)(d->workspace ? d->workspace_bytes : 0));
+  void* const workspace = call.gemm_bytes ? (uint8_t*)d->workspace + call.a_bytes : nullptr;
+  const void* packed_a = a;
+  if (d->a_layout == SMX_A_ROWMAJOR) {
+    packed_a = d->workspace;
+    if (int rc = smx_pack_operand(d->algo, d->formula, d->block_permutation, SMX_SIDE_LHS, d->m, d->k, a, a_dtype,
+                                  passes, d->lda, d->bm, d->bk, nullptr, 0, d->workspace, stream))
+      return rc;
+  } else if (!aligned16(a)) {
+    return fail(SMX_ERR_INVALID, "A must be 16-byte aligned");
+  }
+  call.p.a = (const uint16_t*)packed_a;
+  if (call.stream.shape >= 0) return launch_stream_plan(call.p, call.desc, call.stream, workspace, (hipStream_t)stream);
+  call.desc.workspace = workspace;
+  call.desc.workspace_bytes = call.gemm_bytes;
+  return launch_gemm(call.p, call.desc, (hipStream_t)stream);
 }
 
 int smx_norm_residual_add(int64_t m, int64_t n, const float* x, int64_t ldx, const void* residual, int64_t ldr,

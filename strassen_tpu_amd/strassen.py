@@ -513,12 +513,20 @@ def _run(algo, a, b, *, bm, bn, bk, epilogue=None, residual=None, bias=None,
     _require_device(a.data if isinstance(a, PackedOperand) else a,
                     b.data if isinstance(b, PackedOperand) else b,
                     residual, bias, rope_cos, rope_sin, rope_scale)
+    a_layout, a_dtype = _lib.SMX_A_ROWMAJOR, _lib.SMX_DTYPE_BF16
     if packed:
         if not isinstance(b, PackedOperand):
             b = _plain_weight(b, algo=algo, bn=bn, bk=bk, dot_precision=dot_precision, **variant)
-        if not isinstance(a, PackedOperand):
-            a = pack_operand(a, algo=algo, side="lhs", tile_rows=bm, bk=bk, dot_precision=dot_precision, **variant)
-        a_ptr, b_ptr, lda, ldb = a.data, b.data, k * passes, k * passes
+        if isinstance(a, PackedOperand):
+            a_layout = _lib.SMX_A_PACKED
+            a_ptr, lda = a.data, k * passes
+        else:  # packed by the call itself (smx_matmul), from rows of 16-byte chunks
+            if a.stride(1) != 1 or (a.stride(0) * a.element_size()) % 16 or a.data_ptr() % 16:
+                a = a.contiguous()
+            if a.dtype == torch.float32:
+                a_dtype = _lib.SMX_DTYPE_F32
+            a_ptr, lda = a, a.stride(0)
+        b_ptr, ldb = b.data, k * passes
     else:
         if a.stride(1) != 1 or a.stride(0) % 8 or a.data_ptr() % 16:
             a = a.contiguous()
@@ -534,7 +542,7 @@ def _run(algo, a, b, *, bm, bn, bk, epilogue=None, residual=None, bias=None,
     desc.bm, desc.bn, desc.bk = bm, bn, bk
     desc.algo = algo
     desc.epilogue = _lib.SMX_EPI[epilogue]
-    desc.a_layout = _lib.SMX_A_PACKED if packed else _lib.SMX_A_ROWMAJOR
+    desc.a_layout = a_layout
     desc.b_layout = b_layout
     desc.flags = _lib.SMX_FLAG_OUT_F32 if out_dtype == torch.float32 else 0
     if algo == 7 and packed and STRASSEN_KERNEL == "product_major":
@@ -573,20 +581,22 @@ def _run(algo, a, b, *, bm, bn, bk, epilogue=None, residual=None, bias=None,
         if rope_scale.dtype == torch.float32:
             aux |= _lib.SMX_AUX_SCALE_F32
     desc.aux_f32 = aux
-    # The library asks for a workspace when the tiles of a partly filled last
-    # round run as K shares (FP32 shares of the output, summed by a second
-    # pass) or when the product-major kernel takes the call (its two parked
+    # The library packs a row-major activation into the workspace, and asks
+    # for more of it when K is divided (FP32 shares of the output, summed by a
+    # second pass) or the product-major kernel takes the call (its two parked
     # FP32 sets per tile).
+    stream = torch.cuda.current_stream(a.device).cuda_stream
+    pointers = (_lib.ptr(a_ptr), _lib.ptr(b_ptr), _lib.ptr(c), _lib.ptr(residual), _lib.ptr(bias), _lib.ptr(rope_cos),
+                _lib.ptr(rope_sin), _lib.ptr(rope_scale), stream)
     need = ctypes.c_int64()
-    _lib.check(lib.smx_gemm_workspace_bytes(desc, ctypes.byref(need)))
-    workspace = None
+    if not packed:
+        _lib.check(lib.smx_gemm(desc, *pointers))
+        return c
+    _lib.check(lib.smx_matmul_workspace_bytes(desc, a_dtype, passes, ctypes.byref(need)))
     if need.value:
         workspace = torch.empty(need.value, dtype=torch.uint8, device=a.device)
         desc.workspace, desc.workspace_bytes = workspace.data_ptr(), need.value
-    stream = torch.cuda.current_stream(a.device).cuda_stream
-    rc = lib.smx_gemm(desc, _lib.ptr(a_ptr), _lib.ptr(b_ptr), _lib.ptr(c), _lib.ptr(residual),
-                      _lib.ptr(bias), _lib.ptr(rope_cos), _lib.ptr(rope_sin),
-                      _lib.ptr(rope_scale), stream)
+    rc = lib.smx_matmul(desc, a_dtype, passes, *pointers)
     _lib.check(rc)
     return c
 

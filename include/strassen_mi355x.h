@@ -304,6 +304,16 @@ int smx_pack_operand(int32_t algo, int32_t formula, int32_t block_permutation, i
                      int32_t bk, const int32_t* panels, int64_t src_k, void* out, void* stream);
 
 /*
+ * smx_pack_operand for a right operand whose source is B stored row-major
+ * [k, rows = n] (row stride ld >= n, any alignment of the rows; 16-byte-aligned
+ * rows pack fastest), such as an output gradient. The packed result is that
+ * of SMX_SIDE_RHS on the same B.
+ */
+int smx_pack_rhs_transposed(int32_t algo, int32_t formula, int32_t block_permutation, int64_t rows, int64_t k,
+                            const void* src, int32_t src_dtype, int32_t passes, int64_t ld, int32_t tile_rows,
+                            int32_t bk, const int32_t* panels, int64_t src_k, void* out, void* stream);
+
+/*
  * Second pass of the norm_residual_add epilogue (strassen_pallas.py:836-866),
  * whose norm spans a whole output row: from the FP32 product x [m, n] (an
  * smx_gemm with SMX_FLAG_OUT_F32 and no epilogue) writes

@@ -59,7 +59,7 @@ SMX_QK_SCALE_F32 = 1
 SMX_QK_OUT_F32 = 4
 
 EXPORTS = ("smx_gemm", "smx_gemm_noalloc", "smx_gemm_workspace_bytes", "smx_matmul", "smx_matmul_workspace_bytes",
-           "smx_tile_requirements", "smx_packed_bytes", "smx_pack_operand", "smx_norm_residual_add", "smx_qk_norm_rope", "smx_last_error", "smx_version")
+           "smx_tile_requirements", "smx_packed_bytes", "smx_pack_operand", "smx_pack_rhs_transposed", "smx_norm_residual_add", "smx_qk_norm_rope", "smx_last_error", "smx_version")
 
 
 class SmxGemmDesc(ctypes.Structure):
@@ -113,6 +113,8 @@ def load():
     lib.smx_packed_bytes.restype = ctypes.c_int
     lib.smx_pack_operand.argtypes = [i32, i32, i32, i32, i64, i64, vp, i32, i32, i64, i32, i32, vp, i64, vp, vp]
     lib.smx_pack_operand.restype = ctypes.c_int
+    lib.smx_pack_rhs_transposed.argtypes = [i32, i32, i32, i64, i64, vp, i32, i32, i64, i32, i32, vp, i64, vp, vp]
+    lib.smx_pack_rhs_transposed.restype = ctypes.c_int
     f32 = ctypes.c_float
     lib.smx_norm_residual_add.argtypes = [i64, i64, vp, i64, vp, i64, vp, i32, f32, vp, i64, vp]
     lib.smx_norm_residual_add.restype = ctypes.c_int

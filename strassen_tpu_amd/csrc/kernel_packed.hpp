@@ -329,10 +329,11 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_packed(Params p) {
 
 }
 
-// Packs one operand. kSide 0: A [m, k] row-major (kSide 2: the same A stored
-// transposed as [k, m]), product row R = (tile i,
+// Packs one operand stored with its rows contiguous, [k, rows], whatever its
+// alignment (pack_rows and pack_cols below take the others). kSide 0: A
+// [m, k] (stored [k, m]), product row R = (tile i,
 // row r < bm/2) -> physical rows i*bm + r (top) and + bm/2 (bottom).
-// kSide 1: B^T [n, k] row-major, product column C = (tile j, c < bn/2) ->
+// kSide 1: B^T [n, k] (stored [k, n]), product column C = (tile j, c < bn/2) ->
 // rows j*bn + c (left) and + bn/2 (right) of B^T. Product depth k' = (panel
 // s, kk < bk/2) -> columns s*bk + kk and + bk/2. Quadrants: A0 = (top, k
 // left), A1 = (top, k right), A2 = (bottom, k left), A3 = (bottom, k right);
@@ -340,8 +341,8 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_packed(Params p) {
 // B3 = (k bottom, right) (strassen_pallas.py:188-204). With a panel map,
 // packed K panel s reads source panel panels[s] (the Strassen or the exact
 // panels of an exact-panel schedule); without one, panel s. One wave packs one
-// 32-row product block over kPackStages stages: each lane loads 16 bytes of
-// each quadrant per stage and stores nops 16-byte chunks, so the stores of
+// 32-row product block over kPackStages stages: each lane gathers eight
+// elements of each quadrant per stage and stores nops 16-byte chunks, so the stores of
 // a wave are whole 1 KB fragments.
 // One lane's share of one packed stage: from the four quadrant values x
 // (A: [row half][K half]; B: [K half][column half]) of its 8 consecutive k,
@@ -354,7 +355,7 @@ __device__ __forceinline__ void store_fragments(F8 (&x)[4], int formula, int per
   };
   if constexpr (kAlgo == 7) {
     F8 ops[7];
-    if constexpr (kSide != 1) {
+    if constexpr (kSide == 0) {
       permute_quadrants(x, perm & 1, (perm >> 1) & 1);  // A: (rows, K halves)
       formula_vals<0, !kF32>(formula, x, ops);
     } else {
@@ -396,29 +397,10 @@ __global__ __launch_bounds__(256) void pack_operand(const void* __restrict__ src
   // (their source rows are clamped to row 0 and the values replaced).
   const bool pad = r >= rows / 2;
   const int64_t row_first = pad ? 0 : (r / hr) * tile_rows + r % hr, row_second = row_first + hr;
-  const Elem* const first = src + row_first * ld;
-  const Elem* const second = first + (int64_t)hr * ld;
-  // Eight consecutive elements (columns col0 .. col0+7) of a row-major row.
-  auto load_row = [&](const Elem* row, int64_t col0) {
-    F8 f;
-    if constexpr (kF32) {
-      const f32x4 v0 = *reinterpret_cast<const f32x4*>(row + col0);
-      const f32x4 v1 = *reinterpret_cast<const f32x4*>(row + col0 + 4);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        f.v[e] = v0[e];
-        f.v[4 + e] = v1[e];
-      }
-    } else {
-      f = unpack8(*reinterpret_cast<const u32x4*>(row + col0));
-    }
-    return f;
-  };
-  // kSide 2: A stored transposed, [k, rows] with row stride ld; element
-  // (row, col) of A is src[col * ld + row]. Eight consecutive k of one row
-  // are gathered from eight source rows (lanes cover consecutive rows, so
-  // each load instruction reads 64 contiguous bytes of one source row, 128
-  // for float).
+  // The source is [k, rows] with row stride ld: element (row, col) is
+  // src[col * ld + row]. Eight consecutive k of one row are gathered from
+  // eight source rows (lanes cover consecutive rows, so each load
+  // instruction reads 64 contiguous bytes of one source row, 128 for float).
   auto gather = [&](int64_t row, int64_t col0) {
     F8 f;
 #pragma unroll
@@ -451,104 +433,214 @@ __global__ __launch_bounds__(256) void pack_operand(const void* __restrict__ src
       for (int q = 0; q < 4; ++q)
 #pragma unroll
         for (int e = 0; e < 8; ++e) x[q].v[e] = 0.0f;
-    } else if constexpr (kSide == 2) {
-      x[0] = gather(row_first, lo);
-      x[1] = gather(row_first, hi);
-      x[2] = gather(row_second, lo);
-      x[3] = gather(row_second, hi);
-    } else if constexpr (kSide == 0) {
-      x[0] = load_row(first, lo);
-      x[1] = load_row(first, hi);
-      x[2] = load_row(second, lo);
-      x[3] = load_row(second, hi);
     } else {
-      x[0] = load_row(first, lo);
-      x[1] = load_row(second, lo);
-      x[2] = load_row(first, hi);
-      x[3] = load_row(second, hi);
+      x[0] = gather(row_first, lo);
+      x[kSide == 0 ? 1 : 2] = gather(row_first, hi);
+      x[kSide == 0 ? 2 : 1] = gather(row_second, lo);
+      x[3] = gather(row_second, hi);
     }
     store_fragments<kAlgo, kSide, kF32>(x, formula, perm, part, dst_tile + st * (int64_t)(nops * kBlocks * kFrag));
   }
 }
 
-// pack_operand for bf16 row-major sources (A [rows, k], or a weight stored
-// [n, k]) at one pass, with coalesced reads. pack_operand's lanes read 32
-// source rows per instruction, 32 bytes of each; here a workgroup first
-// copies, for 32 product rows and kRowStages stages, the four source
-// segments of each product row (first / second source row x lower / upper
-// K half, 16 k per stage) into LDS, 16 threads per contiguous 256-byte run.
-// Each wave then forms whole stages from LDS exactly as pack_operand does.
-// The row stride carries a 16-byte pad, so the 8 lanes of one LDS read
-// phase (consecutive rows) fall in distinct banks.
-constexpr int kRowStages = 8;
-constexpr int kRowRun = kRowStages * TK * 2;   // bytes of one segment: 16 k per stage
-constexpr int kRowStride = 4 * kRowRun + 16;  // LDS bytes per product row
+// The packers below copy, for 32 product rows and kStages stages, the four
+// source segments of each product row (first / second source row x lower /
+// upper K half, 16 k per stage) into LDS and form the fragments from there;
+// pack_operand's lanes, which gather straight from the source, read 32 to 64
+// bytes of a row per instruction.
+//
+// A workgroup's place: 32-row product block, first stage, and the geometry
+// of the source, in 32-bit (the host refuses larger operands).
+struct PackGeom {
+  uint32_t rows, tile_rows, hr, bk, hk;
+  uint32_t nsrc;  // stages of one pass: K / (32 passes)
 
+  // Source row of product row r (its second row is hr further).
+  __device__ __forceinline__ uint32_t source_row(uint32_t r) const { return (r / hr) * tile_rows + r % hr; }
+  // First source column of the lower K half of stage st; the upper half is hk
+  // further. A stage's 16 k never cross a panel half (hk is a multiple of
+  // 32). Map entries are clamped to the source, so a bad map cannot read out
+  // of bounds.
+  __device__ __forceinline__ int64_t source_col(uint32_t st, const int32_t* panels, int32_t src_panels) const {
+    const uint32_t kp = st * TK, panel = kp / hk;
+    const int64_t src_panel = panels ? min(max(panels[panel], 0), src_panels - 1) : (int32_t)panel;
+    return src_panel * bk + (kp - panel * hk);
+  }
+};
+
+// LDS bytes of one product row's four segments: kStages x 16 elements each,
+// and a 16-byte pad that puts the 8 lanes of one LDS read phase (consecutive
+// rows) in distinct banks.
+template <int kElem, int kStages>
+constexpr int kPackRow = 4 * kStages * TK * kElem + 16;
+
+// store_fragments of a float source in every pass of a multi-pass product,
+// pass_bytes apart: the operands and their bf16 parts are formed once.
 template <int kAlgo, int kSide>
-__global__ __launch_bounds__(256) void pack_rows(const uint16_t* __restrict__ src, int64_t ld, int64_t rows,
-                                                 int64_t k, int32_t tile_rows, int32_t bk, int32_t formula,
-                                                 int32_t perm, const int32_t* __restrict__ panels,
-                                                 int32_t src_panels, uint8_t* __restrict__ out) {
-  static_assert(kSide == 0 || kSide == 1, "row-major sources only");
-  static_assert(kRowStages % 4 == 0, "whole stages per wave");
-  __shared__ __attribute__((aligned(16))) uint8_t tile[32 * kRowStride];
-  constexpr int nops = nops_of(kAlgo);
-  const int64_t nstages = k / (2 * TK);
-  const int64_t sgroups = (nstages + kRowStages - 1) / kRowStages;
-  const int64_t rblock = blockIdx.x / sgroups;  // 32-row product block
-  if (rblock >= padded_product_rows(rows) / 32) return;  // uniform per workgroup
-  const int64_t st0 = (blockIdx.x - rblock * sgroups) * kRowStages;
-  const int hr = tile_rows / 2, hk = bk / 2;
-  // Copy: 32 rows x 4 segments x kRowStages stages x two 16-byte pieces.
-  constexpr int kPieces = 32 * 4 * kRowStages * 2;
-  static_assert(kPieces % 256 == 0, "whole copy rounds");
-#pragma unroll
-  for (int i = 0; i < kPieces / 256; ++i) {
-    const int piece = i * 256 + (int)threadIdx.x;
-    const int sub = piece & 1, j = (piece >> 1) % kRowStages, rs = (piece >> 1) / kRowStages;
-    const int row = rs >> 2, seg = rs & 3;  // seg bit 1: second source row; bit 0: upper K half
-    const int64_t st = st0 + j;
-    if (st < nstages) {
-      const int64_t r = rblock * 32 + row;
-      uint8_t* const to = tile + row * kRowStride + seg * kRowRun + j * 32 + sub * 16;
-      if (r >= rows / 2) {  // padding of the last 128-row product tile: zeros
-        *reinterpret_cast<u32x4*>(to) = u32x4{0u, 0u, 0u, 0u};
-        continue;
-      }
-      const int64_t srow = (r / hr) * tile_rows + r % hr + ((seg & 2) ? hr : 0);
-      // A stage's 16 k never cross a panel half (hk is a multiple of 32).
-      const int64_t kp = st * TK;
-      const int64_t panel = kp / hk;
-      // Map entries are clamped to the source, so a bad map cannot read out of bounds.
-      const int64_t src_panel = panels ? min(max(panels[panel], 0), src_panels - 1) : panel;
-      const int64_t col = src_panel * bk + kp % hk + ((seg & 1) ? hk : 0) + sub * 8;
-      *reinterpret_cast<u32x4*>(to) = *reinterpret_cast<const u32x4*>(src + srow * ld + col);
+__device__ __forceinline__ void store_passes(F8 (&x)[4], int formula, int perm, int passes, uint8_t* dst,
+                                             int64_t pass_bytes) {
+  auto store = [&](int op, const F8& v) __attribute__((always_inline)) {
+    const u32x4 p0 = pack8_part(v, 0);
+    u32x4 p1 = p0, p2 = p0;
+    if (passes > 1) p1 = pack8_part(v, 1);
+    if (passes > 3) p2 = pack8_part(v, 2);
+    uint8_t* to = dst + op * kBlocks * kFrag;
+    for (int pass = 0; pass < passes; ++pass, to += pass_bytes) {
+      const int part = pass_part(kSide == 1, passes, pass);
+      *reinterpret_cast<u32x4*>(to) = part == 0 ? p0 : part == 1 ? p1 : p2;
     }
-  }
-  __syncthreads();
-  const int wave = (int)threadIdx.x >> 6, lane = (int)threadIdx.x & 63;
-  const uint8_t* const from = tile + (lane & 31) * kRowStride + (lane >> 5) * 16;
-  uint8_t* const dst_tile = out + frag_offset(rblock / 4, 0, nstages, 0, nops, (int)(rblock % 4)) + lane * 16;
-#pragma unroll
-  for (int jj = 0; jj < kRowStages / 4; ++jj) {
-    const int j = jj * 4 + wave;
-    const int64_t st = st0 + j;
-    if (st >= nstages) break;
-    auto seg = [&](int sg) { return unpack8(*reinterpret_cast<const u32x4*>(from + sg * kRowRun + j * 32)); };
-    F8 x[4];
+  };
+  if constexpr (kAlgo == 7) {
+    F8 ops[7];
     if constexpr (kSide == 0) {
-      x[0] = seg(0);  // first row, lower K half
-      x[1] = seg(1);  // first row, upper K half
-      x[2] = seg(2);  // second row, lower K half
-      x[3] = seg(3);  // second row, upper K half
+      permute_quadrants(x, perm & 1, (perm >> 1) & 1);  // A: (rows, K halves)
     } else {
-      x[0] = seg(0);
-      x[1] = seg(2);
-      x[2] = seg(1);
-      x[3] = seg(3);
+      permute_quadrants(x, (perm >> 1) & 1, (perm >> 2) & 1);  // B: (K halves, columns)
     }
-    store_fragments<kAlgo, kSide, false>(x, formula, perm, 0, dst_tile + st * (int64_t)(nops * kBlocks * kFrag));
+    formula_vals<kSide, false>(formula, x, ops);
+#pragma unroll
+    for (int op = 0; op < 7; ++op) store(op, ops[op]);
+  } else {
+#pragma unroll
+    for (int op = 0; op < 4; ++op) store(op, x[op]);
   }
+}
+
+// Stages st0 .. of product block rblock from LDS to `out`, in every pass:
+// wave w forms stages w, w + 4, ...
+template <int kAlgo, int kSide, bool kF32, int kStages>
+__device__ __forceinline__ void pack_from_lds(const uint8_t* tile, uint32_t rblock, uint32_t st0, const PackGeom& g,
+                                              int32_t formula, int32_t perm, int32_t passes, uint8_t* out) {
+  constexpr int kElem = kF32 ? 4 : 2, kRun = kStages * TK * kElem, nops = nops_of(kAlgo);
+  const int wave = (int)threadIdx.x >> 6, lane = (int)threadIdx.x & 63;
+  const uint8_t* const from = tile + (lane & 31) * kPackRow<kElem, kStages> + (lane >> 5) * 8 * kElem;
+  const int64_t nstages = (int64_t)g.nsrc * passes;
+  uint8_t* const dst = out + frag_offset(rblock / 4, 0, nstages, 0, nops, (int)(rblock % 4)) + lane * 16;
+#pragma unroll
+  for (int jj = 0; jj < kStages / 4; ++jj) {
+    const int j = jj * 4 + wave;
+    const uint32_t st = st0 + j;
+    if (st >= g.nsrc) break;
+    auto seg = [&](int sg) __attribute__((always_inline)) {
+      const uint8_t* const at = from + sg * kRun + j * TK * kElem;
+      if constexpr (kF32) {
+        const f32x4 lo = *reinterpret_cast<const f32x4*>(at), hi = *reinterpret_cast<const f32x4*>(at + 16);
+        return F8{{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]}};
+      } else {
+        return unpack8(*reinterpret_cast<const u32x4*>(at));
+      }
+    };
+    // A: (first row, lower K half), (first, upper), (second, lower), (second,
+    // upper); B has K halves outside.
+    F8 x[4] = {seg(0), seg(kSide == 0 ? 1 : 2), seg(kSide == 0 ? 2 : 1), seg(3)};
+    uint8_t* const at = dst + st * (int64_t)(nops * kBlocks * kFrag);
+    if constexpr (!kF32) {
+      store_fragments<kAlgo, kSide, false>(x, formula, perm, 0, at);
+    } else {
+      store_passes<kAlgo, kSide>(x, formula, perm, passes, at, (int64_t)g.nsrc * (nops * kBlocks * kFrag));
+    }
+  }
+}
+
+// Row-major sources (A [rows, k], or a weight stored [n, k]), bf16 or float:
+// every thread copies one 16-byte piece of each of 32 / (rows a round covers)
+// rows, a fixed place in the run, so its column is found once. kStages 8
+// reads 256-byte runs of bf16; launches with few blocks take 4, for twice the
+// workgroups. HBM bound: 8192 x 25600 bf16 for Strassen in 206 us (5.6 TB/s
+// of reads and writes; a copy reaches 5.1), 1024 x 1024 in 3.1; a float
+// source of 4096 x 4096 in six passes in 82 us, its operands formed once.
+template <int kAlgo, int kSide, bool kF32, int kStages>
+__global__ __launch_bounds__(256, kF32 || kSide == 1 ? 3 : 4) void pack_rows(const void* __restrict__ src_v, int64_t ld, PackGeom g,
+                                                 int32_t formula, int32_t perm, const int32_t* __restrict__ panels,
+                                                 int32_t src_panels, int32_t passes, uint8_t* __restrict__ out) {
+  static_assert(kSide == 0 || kSide == 1, "row-major sources only");
+  static_assert(kStages % 4 == 0, "whole stages per wave");
+  constexpr int kElem = kF32 ? 4 : 2, kRun = kStages * TK * kElem, kPieces = kRun / 16, kRow = kPackRow<kElem, kStages>;
+  constexpr int kRowsPerRound = 256 / (4 * kPieces);
+  static_assert(kRowsPerRound > 0 && kRowsPerRound <= 8 && 32 % kRowsPerRound == 0, "whole copy rounds, at most hr rows");
+  __shared__ __attribute__((aligned(16))) uint8_t tile[32 * kRow];
+  const uint32_t sgroups = (g.nsrc + kStages - 1) / kStages;
+  const uint32_t rblock = blockIdx.x / sgroups, st0 = (blockIdx.x - rblock * sgroups) * kStages;
+  const int piece = (int)threadIdx.x % kPieces, seg = (int)threadIdx.x / kPieces % 4;
+  const int row0 = (int)threadIdx.x / (4 * kPieces);
+  const int in_run = piece * 16 / kElem;  // element of the run: 16 per stage
+  // past the last stage: the last one again (never packed)
+  const uint32_t st = min(st0 + in_run / TK, g.nsrc - 1);
+  const int64_t col = g.source_col(st, panels, src_panels) + ((seg & 1) ? g.hk : 0) + in_run % TK;
+  const uint8_t* const src = reinterpret_cast<const uint8_t*>(src_v) + col * kElem;
+  u32x4 v[32 / kRowsPerRound];
+  // the row's tile and its place in the tile's half, one round's rows (at
+  // most hr) further each time
+  uint32_t r = rblock * 32 + row0, row_tile = r / g.hr, in_half = r - row_tile * g.hr;
+#pragma unroll
+  for (int i = 0; i < 32 / kRowsPerRound; ++i) {
+    // Padding of the last 128-row product tile is zeros; it loads the first
+    // row instead of branching, which would move every row loaded so far.
+    const bool pad = r >= g.rows / 2;
+    const uint32_t row = pad ? 0 : row_tile * g.tile_rows + in_half + ((seg & 2) ? g.hr : 0);
+    const u32x4 x = *reinterpret_cast<const u32x4*>(src + (int64_t)row * ld * kElem);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[i][e] = pad ? 0u : x[e];
+    r += kRowsPerRound;
+    in_half += kRowsPerRound;
+    if (in_half >= g.hr) {
+      in_half -= g.hr;
+      ++row_tile;
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < 32 / kRowsPerRound; ++i)
+    *reinterpret_cast<u32x4*>(tile + (i * kRowsPerRound + row0) * kRow + seg * kRun + piece * 16) = v[i];
+  __syncthreads();
+  pack_from_lds<kAlgo, kSide, kF32, kStages>(tile, rblock, st0, g, formula, perm, passes, out);
+}
+
+// bf16 sources stored with their rows contiguous, [k, rows] (A transposed,
+// or a row-major weight [k, n]): every thread reads eight rows of two
+// adjacent k, and the pairs go to LDS as dwords in the rows' order. Two
+// neighbouring row blocks, which share the 128-byte lines, run one after the
+// other on one XCD. Rows of 16-byte chunks only (ld % 8 == 0). 4096 x 8192
+// for Strassen's B: 29 us (6.4 TB/s; a transposing copy and pack_rows took
+// 165 us).
+template <int kAlgo, int kSide>
+__global__ __launch_bounds__(256) void pack_cols(const uint16_t* __restrict__ src, int64_t ld, PackGeom g,
+                                                 int32_t formula, int32_t perm, const int32_t* __restrict__ panels,
+                                                 int32_t src_panels, uint8_t* __restrict__ out) {
+  constexpr int kStages = 8, kRun = kStages * TK * 2, kRow = kPackRow<2, kStages>;
+  __shared__ __attribute__((aligned(16))) uint8_t tile[32 * kRow];
+  const uint32_t sgroups = (g.nsrc + kStages - 1) / kStages;
+  const uint32_t rblocks = gridDim.x / sgroups;
+  const uint32_t sg = blockIdx.x / rblocks;
+  uint32_t rblock = blockIdx.x - sg * rblocks;
+  if (rblocks % 16 == 0) rblock = rblock / 16 * 16 + rblock % 8 * 2 + rblock / 8 % 2;
+  const uint32_t st0 = sg * kStages;
+  const int pair = (int)threadIdx.x / 4, piece = (int)threadIdx.x % 4;
+  const uint32_t st = min(st0 + pair / 8, g.nsrc - 1);  // past the last stage: the last one again
+  const int64_t lo = g.source_col(st, panels, src_panels) + pair % 8 * 2;
+  const uint32_t r = rblock * 32 + piece * 8;
+  const bool pad = r >= g.rows / 2;
+  const uint16_t* const first = src + (pad ? 0 : g.source_row(r));
+  u32x4 even[4], odd[4];
+#pragma unroll
+  for (int seg = 0; seg < 4; ++seg) {
+    const uint16_t* const at = first + (lo + ((seg & 1) ? g.hk : 0)) * ld + ((seg & 2) ? g.hr : 0);
+    const u32x4 x0 = *reinterpret_cast<const u32x4*>(at), x1 = *reinterpret_cast<const u32x4*>(at + ld);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      even[seg][e] = pad ? 0u : x0[e];
+      odd[seg][e] = pad ? 0u : x1[e];
+    }
+  }
+#pragma unroll
+  for (int seg = 0; seg < 4; ++seg)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      uint8_t* const to = tile + (piece * 8 + 2 * i) * kRow + seg * kRun + pair * 4;
+      *reinterpret_cast<uint32_t*>(to) = (even[seg][i] & 0xffffu) | (odd[seg][i] << 16);
+      *reinterpret_cast<uint32_t*>(to + kRow) = (even[seg][i] >> 16) | (odd[seg][i] & 0xffff0000u);
+    }
+  __syncthreads();
+  pack_from_lds<kAlgo, kSide, false, kStages>(tile, rblock, st0, g, formula, perm, 1, out);
 }
 
 }  // namespace packed

@@ -164,31 +164,41 @@ int check_variant(int32_t algo, int32_t formula, int32_t perm) {
   return SMX_OK;
 }
 
+// One packing launch. kSide 0: A, 1: B; transposed: the source is stored
+// [k, rows].
 template <int kAlgo, int kSide>
-int launch_pack(const void* src, bool src_f32, int64_t ld, int64_t rows, int64_t k, int32_t tile_rows, int32_t bk,
-                int32_t formula, int32_t perm, const int32_t* panels, int32_t src_panels, int32_t passes,
+int launch_pack(const void* src, bool src_f32, bool transposed, int64_t ld, int64_t rows, int64_t k, int32_t tile_rows,
+                int32_t bk, int32_t formula, int32_t perm, const int32_t* panels, int32_t src_panels, int32_t passes,
                 uint8_t* out, hipStream_t stream) {
-  const int64_t nstages = k / (2 * packed::TK);
-  if constexpr (kSide != 2) {
-    if (!src_f32) {  // bf16 row-major source: the LDS-staged kernel
-      const int64_t blocks =
-          (packed::padded_product_rows(rows) / 32) * ((nstages + packed::kRowStages - 1) / packed::kRowStages);
-      if (blocks >= ((int64_t)1 << 31)) return fail(SMX_ERR_UNSUPPORTED, "operand too large to pack");
-      hipLaunchKernelGGL((packed::pack_rows<kAlgo, kSide>), dim3((unsigned)blocks), dim3(256), 0, stream,
-                         (const uint16_t*)src, ld, rows, k, tile_rows, bk, formula, perm, panels, src_panels, out);
+  const int64_t nstages = k / (2 * packed::TK), nsrc = nstages / passes;
+  const int64_t rblocks = packed::padded_product_rows(rows) / 32;
+  auto blocks_of = [&](int stages) { return rblocks * ((nsrc + stages - 1) / stages); };
+  constexpr int64_t kMax = (int64_t)1 << 31;
+  if (blocks_of(4) >= kMax || rows >= kMax || k >= kMax) return fail(SMX_ERR_UNSUPPORTED, "operand too large to pack");
+  const packed::PackGeom g{(uint32_t)rows, (uint32_t)tile_rows, (uint32_t)tile_rows / 2, (uint32_t)bk,
+                           (uint32_t)bk / 2, (uint32_t)nsrc};
+  if (transposed) {
+    if (!src_f32 && ld % 8 == 0) {
+      hipLaunchKernelGGL((packed::pack_cols<kAlgo, kSide>), dim3((unsigned)blocks_of(8)), dim3(256), 0, stream,
+                         (const uint16_t*)src, ld, g, formula, perm, panels, src_panels, out);
       return check_launch();
     }
+    const int64_t waves = rblocks * ((nstages + packed::kPackStages - 1) / packed::kPackStages);
+    auto kern = src_f32 ? packed::pack_operand<kAlgo, kSide, true> : packed::pack_operand<kAlgo, kSide, false>;
+    hipLaunchKernelGGL(kern, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, stream, src, ld, rows, k, tile_rows, bk,
+                       formula, perm, panels, src_panels, passes, out);
+    return check_launch();
   }
-  const int64_t waves =
-      (packed::padded_product_rows(rows) / 32) * ((nstages + packed::kPackStages - 1) / packed::kPackStages);
-  const int64_t blocks = (waves + 3) / 4;
-  if (blocks >= ((int64_t)1 << 31)) return fail(SMX_ERR_UNSUPPORTED, "operand too large to pack");
-  if (src_f32)
-    hipLaunchKernelGGL((packed::pack_operand<kAlgo, kSide, true>), dim3((unsigned)blocks), dim3(256), 0, stream, src,
-                       ld, rows, k, tile_rows, bk, formula, perm, panels, src_panels, passes, out);
-  else
-    hipLaunchKernelGGL((packed::pack_operand<kAlgo, kSide, false>), dim3((unsigned)blocks), dim3(256), 0, stream, src,
-                       ld, rows, k, tile_rows, bk, formula, perm, panels, src_panels, 1, out);
+  if (src_f32) {
+    hipLaunchKernelGGL((packed::pack_rows<kAlgo, kSide, true, 4>), dim3((unsigned)blocks_of(4)), dim3(256), 0, stream,
+                       src, ld, g, formula, perm, panels, src_panels, passes, out);
+    return check_launch();
+  }
+  // Below two workgroups of eight stages per CU, half as many stages each.
+  const bool small = blocks_of(8) < 512;
+  auto kern = small ? packed::pack_rows<kAlgo, kSide, false, 4> : packed::pack_rows<kAlgo, kSide, false, 8>;
+  hipLaunchKernelGGL(kern, dim3((unsigned)blocks_of(small ? 4 : 8)), dim3(256), 0, stream, src, ld, g, formula, perm,
+                     panels, src_panels, 1, out);
   return check_launch();
 }
 
@@ -922,21 +932,18 @@ int smx_packed_bytes(int32_t algo, int64_t rows, int64_t k, int64_t* bytes) {
   return SMX_OK;
 }
 
-int smx_pack_operand(int32_t algo, int32_t formula, int32_t block_permutation, int32_t side, int64_t rows, int64_t k,
-                     const void* src, int32_t src_dtype, int32_t passes, int64_t ld, int32_t tile_rows,
-                     int32_t bk, const int32_t* panels, int64_t src_k, void* out, void* stream) {
-  g_error[0] = 0;
+static int pack_any(int32_t algo, int32_t formula, int32_t block_permutation, bool rhs, bool transposed, int64_t rows,
+                    int64_t k, const void* src, int32_t src_dtype, int32_t passes, int64_t ld, int32_t tile_rows,
+                    int32_t bk, const int32_t* panels, int64_t src_k, void* out, void* stream) {
   if (algo != SMX_ALGO_STRASSEN && algo != SMX_ALGO_CUBIC) return fail(SMX_ERR_INVALID, "algo must be 7 or 8");
   if (int rc = check_variant(algo, formula, block_permutation)) return rc;
-  if (side != SMX_SIDE_LHS && side != SMX_SIDE_RHS && side != SMX_SIDE_LHS_T)
-    return fail(SMX_ERR_INVALID, "side must be LHS (0), RHS (1) or LHS_T (2)");
   if (rows <= 0 || k <= 0 || tile_rows <= 0 || bk <= 0 || rows % tile_rows || k % bk)
     return fail(SMX_ERR_INVALID, "packing needs rows %% tile_rows == 0 and K %% bk == 0");
   // A's tile rows may be thin (ThinRows); B's must fill whole product tiles.
-  const int32_t row_granule = side == SMX_SIDE_RHS ? 2 * packed::TN : 2 * kThinRowGranule;
+  const int32_t row_granule = rhs ? 2 * packed::TN : 2 * kThinRowGranule;
   if (tile_rows % row_granule || bk % (2 * packed::kKGranule))
     return fail(SMX_ERR_UNSUPPORTED, "packed tiles need %s %% %d == 0 and bk %% %d == 0 (got %d, %d)",
-                side == SMX_SIDE_RHS ? "bn" : "bm", row_granule, 2 * packed::kKGranule, tile_rows, bk);
+                rhs ? "bn" : "bm", row_granule, 2 * packed::kKGranule, tile_rows, bk);
   if (!src || !out) return fail(SMX_ERR_INVALID, "null pointer");
   if (!aligned16(src) || !aligned16(out)) return fail(SMX_ERR_INVALID, "pointers must be 16-byte aligned");
   if (src_dtype != SMX_DTYPE_BF16 && src_dtype != SMX_DTYPE_F32)
@@ -951,21 +958,32 @@ int smx_pack_operand(int32_t algo, int32_t formula, int32_t block_permutation, i
   if (src_k <= 0 || src_k % bk || src_k / bk >= ((int64_t)1 << 31))
     return fail(SMX_ERR_INVALID, "the source K (%lld) must be a positive multiple of bk", (long long)src_k);
   // Row-major sources are read 16 bytes at a time: rows must stay 16-byte aligned.
-  if (side == SMX_SIDE_LHS_T ? ld < rows : (ld < src_k || ld % (src_f32 ? 4 : 8)))
-    return fail(SMX_ERR_INVALID, side == SMX_SIDE_LHS_T ? "ld must be >= rows for a transposed A"
-                                                        : "ld must be >= K and a multiple of 16 bytes");
-  const void* s16 = src;
-  uint8_t* o8 = (uint8_t*)out;
-  hipStream_t st = (hipStream_t)stream;
+  if (transposed ? ld < rows : (ld < src_k || ld % (src_f32 ? 4 : 8)))
+    return fail(SMX_ERR_INVALID, transposed ? "ld must be >= rows for a transposed source"
+                                            : "ld must be >= K and a multiple of 16 bytes");
   const int32_t sp = (int32_t)(src_k / bk);
-  if (algo == SMX_ALGO_STRASSEN) {
-    if (side == SMX_SIDE_LHS) return launch_pack<7, 0>(s16, src_f32, ld, rows, k, tile_rows, bk, formula, block_permutation, panels, sp, passes, o8, st);
-    if (side == SMX_SIDE_RHS) return launch_pack<7, 1>(s16, src_f32, ld, rows, k, tile_rows, bk, formula, block_permutation, panels, sp, passes, o8, st);
-    return launch_pack<7, 2>(s16, src_f32, ld, rows, k, tile_rows, bk, formula, block_permutation, panels, sp, passes, o8, st);
-  }
-  if (side == SMX_SIDE_LHS) return launch_pack<8, 0>(s16, src_f32, ld, rows, k, tile_rows, bk, formula, block_permutation, panels, sp, passes, o8, st);
-  if (side == SMX_SIDE_RHS) return launch_pack<8, 1>(s16, src_f32, ld, rows, k, tile_rows, bk, formula, block_permutation, panels, sp, passes, o8, st);
-  return launch_pack<8, 2>(s16, src_f32, ld, rows, k, tile_rows, bk, formula, block_permutation, panels, sp, passes, o8, st);
+  auto launch = algo == SMX_ALGO_STRASSEN ? (rhs ? launch_pack<7, 1> : launch_pack<7, 0>)
+                                          : (rhs ? launch_pack<8, 1> : launch_pack<8, 0>);
+  return launch(src, src_f32, transposed, ld, rows, k, tile_rows, bk, formula, block_permutation, panels, sp, passes,
+                (uint8_t*)out, (hipStream_t)stream);
+}
+
+int smx_pack_operand(int32_t algo, int32_t formula, int32_t block_permutation, int32_t side, int64_t rows, int64_t k,
+                     const void* src, int32_t src_dtype, int32_t passes, int64_t ld, int32_t tile_rows,
+                     int32_t bk, const int32_t* panels, int64_t src_k, void* out, void* stream) {
+  g_error[0] = 0;
+  if (side != SMX_SIDE_LHS && side != SMX_SIDE_RHS && side != SMX_SIDE_LHS_T)
+    return fail(SMX_ERR_INVALID, "side must be LHS (0), RHS (1) or LHS_T (2)");
+  return pack_any(algo, formula, block_permutation, side == SMX_SIDE_RHS, side == SMX_SIDE_LHS_T, rows, k, src,
+                  src_dtype, passes, ld, tile_rows, bk, panels, src_k, out, stream);
+}
+
+int smx_pack_rhs_transposed(int32_t algo, int32_t formula, int32_t block_permutation, int64_t rows, int64_t k,
+                            const void* src, int32_t src_dtype, int32_t passes, int64_t ld, int32_t tile_rows,
+                            int32_t bk, const int32_t* panels, int64_t src_k, void* out, void* stream) {
+  g_error[0] = 0;
+  return pack_any(algo, formula, block_permutation, true, true, rows, k, src, src_dtype, passes, ld, tile_rows, bk,
+                  panels, src_k, out, stream);
 }
 
 int smx_gemm(const smx_gemm_desc* d, const void* a, const void* b, void* c, const void* residual, const void* bias,

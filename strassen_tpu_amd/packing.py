@@ -201,21 +201,24 @@ def packed_bytes(algo, rows, k):
 
 
 def _pack(src, *, algo, side, rows, k, tile_rows, bk, formula, block_permutation, panels=None, passes=1):
-    """One smx_pack_operand call over ``src`` (rows x K source, or K x rows
-    for lhs_t); ``panels`` (a device int32 map) selects the K panels to
+    """One packing call over ``src`` (rows x K source, or K x rows for lhs_t
+    and rhs_t); ``panels`` (a device int32 map) selects the K panels to
     pack, in order; ``passes`` > 1 packs the bf16 parts of a multi-pass
     product after each panel."""
     packed_k = k if panels is None else panels.numel() * bk
     nbytes = packed_bytes(algo, rows, packed_k * passes)
     data = torch.empty(nbytes // 2, dtype=torch.bfloat16, device=src.device)
-    side_id = {"lhs": _lib.SMX_SIDE_LHS, "rhs": _lib.SMX_SIDE_RHS, "lhs_t": _lib.SMX_SIDE_LHS_T}[side]
     stream = torch.cuda.current_stream(src.device).cuda_stream
     src_dtype = _lib.SMX_DTYPE_F32 if src.dtype == torch.float32 else _lib.SMX_DTYPE_BF16
-    rc = _lib.load().smx_pack_operand(algo, _lib.SMX_FORMULA[formula], block_permutation, side_id, rows,
-                                      packed_k * passes, _lib.ptr(src), src_dtype, passes, src.stride(0), tile_rows,
-                                      bk, _lib.ptr(panels), k, _lib.ptr(data), stream)
+    source = (rows, packed_k * passes, _lib.ptr(src), src_dtype, passes, src.stride(0), tile_rows, bk,
+              _lib.ptr(panels), k, _lib.ptr(data), stream)
+    if side == "rhs_t":
+        rc = _lib.load().smx_pack_rhs_transposed(algo, _lib.SMX_FORMULA[formula], block_permutation, *source)
+    else:
+        side_id = {"lhs": _lib.SMX_SIDE_LHS, "rhs": _lib.SMX_SIDE_RHS, "lhs_t": _lib.SMX_SIDE_LHS_T}[side]
+        rc = _lib.load().smx_pack_operand(algo, _lib.SMX_FORMULA[formula], block_permutation, side_id, *source)
     _lib.check(rc)
-    return PackedOperand(data, algo=algo, side="rhs" if side == "rhs" else "lhs", rows=rows, k=packed_k,
+    return PackedOperand(data, algo=algo, side="rhs" if side in ("rhs", "rhs_t") else "lhs", rows=rows, k=packed_k,
                          tile_rows=tile_rows, bk=bk, formula=formula, block_permutation=block_permutation,
                          source_dtype=src.dtype, passes=passes)
 
@@ -225,7 +228,8 @@ def pack_operand(x, *, algo, side, tile_rows, bk, formula="classical", block_per
     """Pack ``x`` (bf16 on the HIP device): ``a [M, K]`` for ``side="lhs"``,
     the same ``a`` stored transposed as ``[K, M]`` for ``side="lhs_t"``, or a
     weight ``b [K, N]`` for ``side="rhs"`` (any strides; a K-contiguous view
-    of ``[N, K]`` storage is read in place). Runs asynchronously on torch's
+    of ``[N, K]`` storage and a row-major ``[K, N]`` with 16-byte-aligned rows
+    are read in place). Runs asynchronously on torch's
     current stream. Strassen operands carry the operand sums of
     ``formula`` ("classical", "dual" or "powers") after the quadrant swaps of
     ``block_permutation``; both operands of a GEMM must be packed alike. With
@@ -253,7 +257,10 @@ def pack_operand(x, *, algo, side, tile_rows, bk, formula="classical", block_per
     else:
         src = x if side == "lhs" else x.t()  # rows x K, K contiguous
         rows, k = src.shape
-        if src.stride(1) != 1 or (src.stride(0) * src.element_size()) % 16 or src.data_ptr() % 16:
+        chunks = x.data_ptr() % 16 == 0 and (x.stride(0) * x.element_size()) % 16 == 0
+        if side == "rhs" and src.stride(1) != 1 and x.stride(1) == 1 and x.stride(0) >= rows and chunks:
+            src, side = x, "rhs_t"  # a row-major [K, N] weight or gradient, read as it lies
+        elif src.stride(1) != 1 or (src.stride(0) * src.element_size()) % 16 or src.data_ptr() % 16:
             src = src.contiguous()
     if rows % tile_rows or k % bk:
         raise ValueError(f"operand [{rows}, {k}] (rows x K) does not tile by ({tile_rows}, {bk})")
@@ -272,7 +279,7 @@ def pack_operand(x, *, algo, side, tile_rows, bk, formula="classical", block_per
                          panels=schedule.panel_map("ordinary", x.device), passes=passes, **common)
     exact = _pack(src, algo=_lib.SMX_ALGO_CUBIC, formula="classical", block_permutation=0,
                   panels=schedule.panel_map("exact", x.device), passes=passes, **common)
-    common["side"] = "rhs" if side == "rhs" else "lhs"
+    common["side"] = "rhs" if side in ("rhs", "rhs_t") else "lhs"
     return SplitOperand(ordinary, exact, formula=formula, block_permutation=block_permutation, schedule=schedule,
                         **common)
 

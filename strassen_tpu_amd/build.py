@@ -123,7 +123,7 @@ def verify_inline_asm_kernels(asm_text):
 # hot path).
 _KERNEL_DESC = re.compile(r"\.amdhsa_kernel (\S+)(.*?)\.end_amdhsa_kernel", re.S)
 _SPLIT = re.compile(r"gemm_splitILi(\d+)ELi(\d+)ELb(\d)E")
-_PM = re.compile(r"gemm_pmILi(\d+)EE")
+_PM = re.compile(r"gemm_pmILi(\d+)ELi(\d+)EE")
 _STREAM = re.compile(r"gemm_streamILi(\d+)E")
 _PACKED = re.compile(r"gemm_packedILi(\d+)ELi(\d+)ELi(\d+)ELi(\d+)ELb(\d)E")
 _QUAD_CUBIC_PARTIAL = 1

@@ -7,7 +7,8 @@ namespace smx {
 
 template <int kEpi>
 int launch_pm_epilogue(const Params& p, hipStream_t stream) {
-  return launch_kernel(pm::gemm_pm<kEpi>, p, p.tiles_m * p.tiles_n, pm::kLds, stream);
+  auto kern = p.k % 256 == 0 ? pm::gemm_pm<kEpi, 8> : pm::gemm_pm<kEpi, pm::kMinSteps>;
+  return launch_kernel(kern, p, p.tiles_m * p.tiles_n, pm::kLds, stream);
 }
 
 int launch_strassen_pm(const Params& p, int epilogue, hipStream_t s) {

@@ -36,20 +36,24 @@
 // reads packed A tile tile_m and packed B tiles 2 tile_n and 2 tile_n + 1,
 // one operand (the current product's) per stage.
 //
-// Pipeline: a stage is 64 product-space k (four packed 16-k stages,
-// "quarters") of one product, 16 KB of A and 32 KB of B; a ring of three
-// stages is refilled two stages ahead, and the DMA stream runs on across
-// product boundaries. One barrier per stage, before its last quarter's
-// MFMAs: it sees the next stage landed and every wave done reading the
-// stage, whose slot the refill then starts on. Per wave and stage: 24
-// fragment reads, 32 MFMAs and 12 DMAs, three per quarter, each issued
-// between two MFMAs (after the second, fifth and eighth of the quarter):
-// DMAs issued back to back hold back the next MFMA's issue (4% on the
-// gate|up launch).
+// Waves: wave w owns all 128 product rows and columns 64 w .. + 63 of the
+// tile, 4 x 2 blocks of 32 x 32 per set; per 16 k it uses 4 A and 2 B
+// fragments for 8 MFMAs. A's fragments are shared by the four waves and go
+// through LDS; B's belong to one wave each and go straight into its
+// registers. LDS then carries 64 KB of reads and 16 KB of DMA writes per
+// 1024 cycles of MFMAs; with both operands in LDS and 64 x 128 waves it was
+// 96 and 48 KB, more than its 128 bytes a cycle. Gate|up call (8192 x 5120 x
+// 51200, SwiGLU): 3.488 -> 3.364 ms, the chip being power limited.
 //
-// Waves: wave (wm, wn) owns product rows 64 wm .. + 63 and columns
-// 128 wn .. + 127 of the tile, 2 x 4 blocks of 32 x 32 per set; per 16 k it
-// reads 2 A and 4 B fragments for 8 MFMAs.
+// Pipeline: a stage is kQ 16-k steps of one product. B is loaded one stage
+// ahead (kQ = 8: 2048 cycles of MFMAs), A's ring is refilled kSlots - 1
+// stages ahead, and both streams run on across product boundaries, except
+// that no B is loaded ahead of an epilogue, which needs its registers. One
+// barrier per stage, before its last step's MFMAs: it sees A's next stage
+// landed and every wave done reading the stage, whose slot the refill then
+// starts on. Each step issues one A DMA and two B loads, each between two
+// MFMAs: VMEM operations issued back to back hold back the next MFMA's issue
+// (4% on the gate|up launch).
 #pragma once
 
 #include "kernel_packed.hpp"
@@ -67,19 +71,22 @@ constexpr int kOps = 7;
 // seven operands: 28 KB.
 constexpr int kOpStage = kBlocks * kFrag;
 constexpr int kPackedStage = kOps * kOpStage;
-// Pipeline stage: four packed 16-k stages ("quarters") of one product; a
-// quarter holds A blocks 0-3, then B tile 0 blocks 0-3, then B tile 1
-// blocks 0-3.
-constexpr int kQuarters = 4;
-constexpr int kQuarterBytes = 3 * kOpStage;            // 12 KB
-constexpr int kStageBytes = kQuarters * kQuarterBytes;  // 48 KB
-constexpr int kSlots = 3;
-constexpr int kDist = kSlots - 1;  // refill distance in stages
-constexpr int kDmaPerWave = kStageBytes / kFrag / 4;  // 12
-// VMEM operations a wave may leave in flight at the barrier of stage g,
-// which needs stage g + 1: the refill of stage g + 2.
-constexpr int kPending = (kDist - 1) * kDmaPerWave;
-constexpr int kRingBytes = kSlots * kStageBytes;
+// Pipeline stage: kQ packed 16-k stages ("steps") of one product, 8 (K a
+// multiple of 256) or 4. A's steps go through a ring of kSlots stages in
+// LDS, refilled kSlots - 1 stages ahead; B's fragments, each read by one
+// wave only, go straight into that wave's registers, one stage ahead.
+constexpr int kMinSteps = 4;
+constexpr int kRingBytes = 128 * 1024;
+template <int kQ>
+struct Ring {
+  static constexpr int kStageBytes = kQ * kOpStage;
+  static constexpr int kSlots = kRingBytes / kStageBytes;
+  // VMEM operations of one wave and stage: one A DMA and two B loads a step.
+  // What a wave may leave in flight at the barrier of stage g, which needs
+  // A's stage g + 1: that was issued kSlots - 2 >= 2 stages before g.
+  static constexpr int kPending = 3 * kQ;
+  static_assert(kSlots >= 4 && kPending < 64, "ring depth and vmcnt range");
+};
 // Epilogue staging tile of a wave: 32 x 32 floats, rows unpadded (the ring
 // leaves 16 KB of the LDS). Same interface as StageTile.
 struct Tile {
@@ -91,7 +98,6 @@ struct Tile {
 };
 constexpr int kLds = kRingBytes + 4 * Tile::kBytes;
 static_assert(kLds <= 160 * 1024, "LDS budget");
-static_assert(kPending < 64, "vmcnt range");
 // One parked set of one workgroup (FP32, 128 x 256), in the registers' lane
 // order: [wave][block][4 register groups][64 lanes][4 floats]; a workgroup
 // parks two.
@@ -103,71 +109,49 @@ constexpr int64_t kParkBytes = 2 * kParkSet;
 constexpr uint32_t kOrder = 4u | 2u << 4 | 3u << 8 | 0u << 12 | 6u << 16 | 5u << 20 | 1u << 24;
 __host__ __device__ constexpr int product_of(int ph) { return (int)((kOrder >> (4 * ph)) & 15u); }
 
-typedef f32x16 Set[2][4];
+// A wave's accumulators of one set: 128 rows x 64 columns.
+constexpr int kRowBlocks = 4, kColBlocks = 2;
+typedef f32x16 Set[kRowBlocks][kColBlocks];
 
-struct Frags {
-  bf16x8 a[2];
-  bf16x8 b[4];
+struct FragsA {
+  bf16x8 v[kRowBlocks];
+};
+struct FragsB {
+  bf16x8 v[kColBlocks];
 };
 
 // File of a set's accumulators: V in VGPRs, A1 and A2 in AGPRs.
 constexpr int kV = 0, kA1 = 1, kA2 = 2;
 __host__ __device__ constexpr bool in_agprs(int set) { return set != kV; }
 
-// The MFMAs of one 16-k half on a set's 2 x 4 blocks. kStart 0: chain
-// (D = A B + D); 1: the product's first half from zero (D = A B); 2: its
-// first half from set `from` of the same file (D = A B + from).
-template <int kSet, int kStart>
-__device__ __forceinline__ void mfma8(Set& acc, const Set& from, const Frags& f) {
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      if constexpr (kStart == 0) {
-        if constexpr (in_agprs(kSet))
-          packed::mfma_agpr(acc[i][j], f.a[i], f.b[j]);
-        else
-          packed::mfma_vgpr(acc[i][j], f.a[i], f.b[j]);
-      } else if constexpr (kStart == 1) {
-        if constexpr (in_agprs(kSet))
-          asm("v_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=&a"(acc[i][j]) : "v"(f.a[i]), "v"(f.b[j]));
-        else
-          asm("v_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=&v"(acc[i][j]) : "v"(f.a[i]), "v"(f.b[j]));
-      } else {
-        static_assert(in_agprs(kSet), "only the AGPR sets start from another set");
-        asm("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %3"
-            : "=&a"(acc[i][j])
-            : "v"(f.a[i]), "v"(f.b[j]), "a"(from[i][j]));
-      }
-    }
-}
-
-// mfma8 with hook(k) after MFMA k (k = 0..7), each hook between scheduling
-// barriers.
+// The MFMAs of one 16-k step on a set's 4 x 2 blocks, column by column, with
+// hook(k) after MFMA k (k = 0..7) between scheduling barriers. kStart 0:
+// chain (D = A B + D); 1: the product's first step from zero (D = A B); 2:
+// its first step from set `from` of the same file (D = A B + from).
 template <int kSet, int kStart, class Hook>
-__device__ __forceinline__ void mfma8_dma(Set& acc, const Set& from, const Frags& f, Hook hook) {
+__device__ __forceinline__ void mfma8(Set& acc, const Set& from, const FragsA& a, const FragsB& b, Hook hook) {
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int j = 0; j < kColBlocks; ++j)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    for (int i = 0; i < kRowBlocks; ++i) {
       if constexpr (kStart == 0) {
         if constexpr (in_agprs(kSet))
-          packed::mfma_agpr(acc[i][j], f.a[i], f.b[j]);
+          packed::mfma_agpr(acc[i][j], a.v[i], b.v[j]);
         else
-          packed::mfma_vgpr(acc[i][j], f.a[i], f.b[j]);
+          packed::mfma_vgpr(acc[i][j], a.v[i], b.v[j]);
       } else if constexpr (kStart == 1) {
         if constexpr (in_agprs(kSet))
-          asm("v_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=&a"(acc[i][j]) : "v"(f.a[i]), "v"(f.b[j]));
+          asm("v_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=&a"(acc[i][j]) : "v"(a.v[i]), "v"(b.v[j]));
         else
-          asm("v_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=&v"(acc[i][j]) : "v"(f.a[i]), "v"(f.b[j]));
+          asm("v_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=&v"(acc[i][j]) : "v"(a.v[i]), "v"(b.v[j]));
       } else {
         static_assert(in_agprs(kSet), "only the AGPR sets start from another set");
         asm("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %3"
             : "=&a"(acc[i][j])
-            : "v"(f.a[i]), "v"(f.b[j]), "a"(from[i][j]));
+            : "v"(a.v[i]), "v"(b.v[j]), "a"(from[i][j]));
       }
       __builtin_amdgcn_sched_barrier(0);
-      hook(4 * i + j);
+      hook(kRowBlocks * j + i);
       __builtin_amdgcn_sched_barrier(0);
     }
 }
@@ -180,9 +164,9 @@ __device__ __forceinline__ void drain(Set& acc) {
   __builtin_amdgcn_sched_barrier(0);
   asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7\n\ts_nop 7" ::: "memory");
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < kRowBlocks; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    for (int j = 0; j < kColBlocks; ++j) {
       if constexpr (in_agprs(kSet))
         asm volatile("" : "+a"(acc[i][j]));
       else
@@ -195,9 +179,9 @@ __device__ __forceinline__ void drain(Set& acc) {
 // region: a uniform base, the lane's 32-bit byte offset (derived where it is
 // used, so no per-lane 64-bit address is held across the main loops) and a
 // compile-time offset. Lane l of register group g of block (i, j) of set x
-// of wave w sits at x kParkSet + w kParkSet / 4 + (4 (4 i + j) + g) KB + 16 l.
+// of wave w sits at x kParkSet + w kParkSet / 4 + (4 (2 i + j) + g) KB + 16 l.
 __device__ __forceinline__ uint32_t park_offset(int set, int wave, int i, int j, int g) {
-  return (uint32_t)(set * kParkSet + wave * (kParkSet / 4) + ((4 * i + j) * 4 + g) * 1024);
+  return (uint32_t)(set * kParkSet + wave * (kParkSet / 4) + ((kColBlocks * i + j) * 4 + g) * 1024);
 }
 
 // Stores x (plus y, when kAdd) as parked set kSetIdx.
@@ -205,9 +189,9 @@ template <int kSetIdx, bool kAdd>
 __device__ __forceinline__ void park_store(__amdgpu_buffer_rsrc_t park, int wave, const Set& x, const Set& y) {
   const uint32_t lane16 = opaque_lane_id() * 16;
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int i = 0; i < kRowBlocks; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int j = 0; j < kColBlocks; ++j)
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
         f32x4 v;
@@ -250,7 +234,6 @@ constexpr int kParkAhead = 2;
 template <int kEpi, int kParks, class Quads>
 __device__ __forceinline__ void emit_half(const Params& p, const TileOrigin& o, int wave, int lr,
                                           __amdgpu_buffer_rsrc_t park, Quads quads, uint8_t* tile) {
-  const int wm = wave >> 1, wn = wave & 1;
   using T = Tile;
   const int lane = opaque_lane_id();
   const int lcol = lane & 31;
@@ -269,17 +252,17 @@ __device__ __forceinline__ void emit_half(const Params& p, const TileOrigin& o, 
   const uint32_t lane16 = lane * 16;
   f32x16 pk[kParkAhead + 1][kParks];
   auto fetch = [&](f32x16 (&to)[kParks], int b) __attribute__((always_inline)) {
-    to[0] = park_block<0>(park, wave, lane16, b >> 2, b & 3);
-    if constexpr (kParks > 1) to[kParks - 1] = park_block<kParks - 1>(park, wave, lane16, b >> 2, b & 3);
+    to[0] = park_block<0>(park, wave, lane16, b / kColBlocks, b % kColBlocks);
+    if constexpr (kParks > 1) to[kParks - 1] = park_block<kParks - 1>(park, wave, lane16, b / kColBlocks, b % kColBlocks);
   };
 #pragma unroll
   for (int f = 0; f < kParkAhead; ++f) fetch(pk[f], f);
 #pragma unroll
   for (int b = 0; b < 8; ++b) {
-    const int i = b >> 2, j = b & 3;
+    const int i = b / kColBlocks, j = b % kColBlocks;
     if (b + kParkAhead < 8) fetch(pk[(b + kParkAhead) % (kParkAhead + 1)], b + kParkAhead);
-    const int64_t row = o.ti * p.bm + o.tr + wm * 64 + i * 32 + half * hm;
-    const int64_t cc = o.tc + wn * 128 + j * 32;  // column inside a column half
+    const int64_t row = o.ti * p.bm + o.tr + i * 32 + half * hm;
+    const int64_t cc = o.tc + wave * 64 + j * 32;  // column inside a column half
     f32x16 left, right;
     quads(i, j, pk[b % (kParkAhead + 1)], left, right);
     if constexpr (kEpi == SMX_EPI_SWIGLU || kEpi == SMX_EPI_GEGLU) {
@@ -319,11 +302,11 @@ __device__ __forceinline__ void emit_half(const Params& p, const TileOrigin& o, 
   }
 }
 
-template <int kEpi>
+template <int kEpi, int kQ>
 __global__ __launch_bounds__(kThreads, 1) void gemm_pm(Params p) {
+  using R = Ring<kQ>;
   extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-  const int wm = wave >> 1, wn = wave & 1;
   int tile_m, tile_n;
   tile_of((int)blockIdx.x, p.tiles_m, p.tiles_n, p.group_m, p.raster, tile_m, tile_n);
   tile_m = __builtin_amdgcn_readfirstlane(tile_m);
@@ -331,119 +314,139 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_pm(Params p) {
   const TileOrigin o = tile_origin<false>(p, (int64_t)tile_m * TM, (int64_t)tile_n * TN);
 
   // Packed 16-k stages over K, and pipeline stages per product (the host
-  // takes K % 128 == 0).
+  // takes K a multiple of 32 kQ).
   const int nst16 = (int)(p.k / 32);
-  const int nstages = nst16 / kQuarters;
+  const int nstages = nst16 / kQ;
   // One packed tile's panel (all stages, all operands); B's second tile
-  // follows its first.
+  // follows its first. Wave w moves block w of A's steps into LDS and loads
+  // its own 64 columns of B: blocks 2 (w % 2) and the next of tile w / 2.
   const uint32_t panel = (uint32_t)nst16 * kPackedStage;
   const __amdgpu_buffer_rsrc_t a_src = packed::panel_rsrc(
       reinterpret_cast<const uint8_t*>(p.a) + (int64_t)tile_m * panel + wave * kFrag, panel - wave * kFrag);
+  const uint32_t b_block = (wave & 1) * kColBlocks * kFrag;
   const __amdgpu_buffer_rsrc_t b_src = packed::panel_rsrc(
-      reinterpret_cast<const uint8_t*>(p.b) + (int64_t)(2 * tile_n) * panel + wave * kFrag, 2 * panel - wave * kFrag);
+      reinterpret_cast<const uint8_t*>(p.b) + (int64_t)(2 * tile_n + (wave >> 1)) * panel + b_block, panel - b_block);
   // The workgroup's parked sets q1 and q3.
   const __amdgpu_buffer_rsrc_t park = packed::panel_rsrc(
       reinterpret_cast<const uint8_t*>(p.park) + (int64_t)blockIdx.x * kParkBytes, (uint32_t)kParkBytes);
   uint8_t* const tile = lds + kRingBytes + wave * Tile::kBytes;
 
-  // DMA x of quarter q of stage (ph, s) into ring slot `slot`: wave w moves
-  // block w of A (x = 0) and of each B tile (x = 1, 2). Stages past the
-  // last one re-load it (in bounds, never read).
-  auto dma_one = [&](int ph, int s, int q, int slot, uint32_t lane_off, int x) __attribute__((always_inline)) {
+  // Byte offset of step q of stage (ph, s) in a panel. Stages past the last
+  // one re-load it (in bounds, never used).
+  auto step_offset = [&](int ph, int s, int q) __attribute__((always_inline)) {
     if (ph >= kOps) {
       ph = kOps - 1;
       s = nstages - 1;
     }
-    const uint32_t off = (uint32_t)((kQuarters * s + q) * kOps + product_of(ph)) * kOpStage;
-    uint8_t* const to = lds + slot * kStageBytes + q * kQuarterBytes + wave * kFrag;
-    if (x == 0) packed::dma_frag(a_src, lane_off, off, to);
-    if (x == 1) packed::dma_frag(b_src, lane_off, off, to + kOpStage);
-    if (x == 2) packed::dma_frag(b_src, lane_off, off + panel, to + 2 * kOpStage);
+    return (uint32_t)((kQ * s + q) * kOps + product_of(ph)) * kOpStage;
   };
-  auto dma_quarter = [&](int ph, int s, int q, int slot, uint32_t lane_off) __attribute__((always_inline)) {
-#pragma unroll
-    for (int x = 0; x < 3; ++x) dma_one(ph, s, q, slot, lane_off, x);
+  auto dma_a = [&](int ph, int s, int q, int slot, uint32_t lane16) __attribute__((always_inline)) {
+    packed::dma_frag(a_src, lane16, step_offset(ph, s, q), lds + slot * R::kStageBytes + q * kOpStage + wave * kFrag);
   };
-  // Hook for mfma8_dma: the three DMAs of quarter q after MFMAs 1, 4 and 7.
-  auto dma_hook = [&](int ph, int s, int q, int slot, uint32_t lane_off) __attribute__((always_inline)) {
-    return [=, &dma_one](int k) __attribute__((always_inline)) {
-      if (k == 1) dma_one(ph, s, q, slot, lane_off, 0);
-      if (k == 4) dma_one(ph, s, q, slot, lane_off, 1);
-      if (k == 7) dma_one(ph, s, q, slot, lane_off, 2);
-    };
+  auto load_b = [&](int ph, int s, int q, int j, uint32_t lane16) __attribute__((always_inline)) {
+    return __builtin_bit_cast(
+        bf16x8, __builtin_amdgcn_raw_buffer_load_b128(b_src, lane16 + j * kFrag, step_offset(ph, s, q), 0));
   };
-  auto load = [&](int slot, int q) __attribute__((always_inline)) {
-    const int lo = opaque_lane_id() * 16;
-    const uint8_t* const base = lds + slot * kStageBytes + q * kQuarterBytes + lo;
-    Frags f;
+  auto read_a = [&](int slot, int q) __attribute__((always_inline)) {
+    const uint8_t* const base = lds + slot * R::kStageBytes + q * kOpStage + opaque_lane_id() * 16;
+    FragsA f;
 #pragma unroll
-    for (int i = 0; i < 2; ++i) f.a[i] = packed::ld_frag(base + (2 * wm + i) * kFrag);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) f.b[j] = packed::ld_frag(base + (4 + 4 * wn + j) * kFrag);
+    for (int i = 0; i < kRowBlocks; ++i) f.v[i] = packed::ld_frag(base + i * kFrag);
     return f;
   };
 
-  // Prologue: stages 0 .. kDist-1 of the stream, and quarter 0 of stage
-  // kDist (the stage loop refills quarters 1-3 of the slot it reads, and
-  // quarter 0 of the next refill after its barrier).
-  int dph = kDist / nstages, ds = kDist % nstages;
+  // Stage counters of the A refill (dph, ds) and of the B loads (bph, bs),
+  // stepped through the products' stages.
+  auto step = [&](int& ph, int& s) __attribute__((always_inline)) {
+    if (++s == nstages) {
+      s = 0;
+      ++ph;
+    }
+  };
+  int dph = 0, ds = 0, bph = 0, bs = 0;
+  FragsB b[kQ];
+  auto load_stage_b = [&]() __attribute__((always_inline)) {
+    const uint32_t lane16 = opaque_lane_id() * 16;
+#pragma unroll
+    for (int q = 0; q < kQ; ++q)
+#pragma unroll
+      for (int j = 0; j < kColBlocks; ++j) b[q].v[j] = load_b(bph, bs, q, j, lane16);
+    step(bph, bs);
+  };
+  // Prologue: A's stage 0, B's stage 0, A's stages 1 .. kSlots - 2, and the
+  // first step of the refill that the stage loop goes on with.
   {
-    const uint32_t lane_off = opaque_lane_id() * 16;
+    const uint32_t lane16 = opaque_lane_id() * 16;
 #pragma unroll
-    for (int st = 0; st < kDist; ++st)
+    for (int st = 0; st < R::kSlots - 1; ++st) {
 #pragma unroll
-      for (int q = 0; q < kQuarters; ++q) dma_quarter(st / nstages, st % nstages, q, st, lane_off);
-    dma_quarter(dph, ds, 0, kDist, lane_off);
+      for (int q = 0; q < kQ; ++q) dma_a(dph, ds, q, st, lane16);
+      step(dph, ds);
+      if (st == 0) load_stage_b();
+    }
+    dma_a(dph, ds, 0, R::kSlots - 1, lane16);
   }
-  packed::stage_barrier<kPending + 3>();
+  packed::stage_barrier<0>();
 
   Set V, A1, A2;
   int slot = 0;
-  Frags cur = load(0, 0);
+  FragsA cur = read_a(0, 0);
 
-  // One pipeline stage: each quarter's fragments read under the previous
-  // quarter's MFMAs; quarters 1-3 of the refill of the slot read at the
-  // previous stage under the first three quarters' MFMAs; the barrier; then
-  // the next stage's first quarter read, and quarter 0 of the refill of the
-  // slot this stage read, under the last quarter's MFMAs. Every wave has
-  // read all of that slot by the barrier (its quarter 0 before the previous
-  // one), and at the barrier a wave leaves only the current refill's 12
-  // DMAs in flight, so the previous refill (the next stage) has landed.
-  // kStart applies to the first quarter (the product's first stage).
-  auto stage = [&](auto setc, auto startc, Set& acc, const Set& from) __attribute__((always_inline)) {
+  // One pipeline stage: each step's A fragments read under the previous
+  // step's MFMAs; behind each step's MFMAs one A DMA of the refill of the
+  // slot read at the previous stage (its steps 1 .. kQ - 1 during the first
+  // kQ - 1 steps) and the step's B fragments of the next stage, one VMEM
+  // operation at a time between two MFMAs. Before the last step the barrier:
+  // every wave has then read all of this stage's slot, whose refill starts
+  // behind it, and A's next stage has landed. kStart applies to the first
+  // step (the product's first stage). kLast: an epilogue follows, which
+  // needs the registers: nothing is loaded ahead.
+  auto stage = [&](auto setc, auto startc, auto lastc, Set& acc, const Set& from) __attribute__((always_inline)) {
     constexpr int kSet = decltype(setc)::value, kStart = decltype(startc)::value;
-    const int next = slot == kSlots - 1 ? 0 : slot + 1;
-    const int fill = slot == 0 ? kSlots - 1 : slot - 1;
-    const uint32_t lane_off = opaque_lane_id() * 16;
+    constexpr bool kLast = decltype(lastc)::value != 0;
+    const int next = slot == R::kSlots - 1 ? 0 : slot + 1;
+    const int fill = slot == 0 ? R::kSlots - 1 : slot - 1;
+    const uint32_t lane16 = opaque_lane_id() * 16;
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int q = 0; q < kQuarters - 1; ++q) {
-      const Frags nxt = load(slot, q + 1);
+    for (int q = 0; q < kQ; ++q) {
+      FragsA nxt{};
+      if (q < kQ - 1) {
+        nxt = read_a(slot, q + 1);
+      } else {
+        step(dph, ds);
+        packed::stage_barrier<R::kPending>();
+        if constexpr (!kLast) nxt = read_a(next, 0);  // past the last stage: a re-loaded copy, unused
+      }
       __builtin_amdgcn_sched_barrier(0);
+      auto hook = [&](int k) __attribute__((always_inline)) {
+        if (k == 1) dma_a(dph, ds, q < kQ - 1 ? q + 1 : 0, q < kQ - 1 ? fill : slot, lane16);
+        if constexpr (!kLast) {
+          if (k == 4) b[q].v[0] = load_b(bph, bs, q, 0, lane16);
+          if (k == 7) b[q].v[1] = load_b(bph, bs, q, 1, lane16);
+        }
+      };
       if (q == 0)
-        mfma8_dma<kSet, kStart>(acc, from, cur, dma_hook(dph, ds, q + 1, fill, lane_off));
+        mfma8<kSet, kStart>(acc, from, cur, b[q], hook);
       else
-        mfma8_dma<kSet, 0>(acc, from, cur, dma_hook(dph, ds, q + 1, fill, lane_off));
-      __builtin_amdgcn_sched_barrier(0);
+        mfma8<kSet, 0>(acc, from, cur, b[q], hook);
       cur = nxt;
     }
-    if (++ds == nstages) {
-      ds = 0;
-      ++dph;
-    }
-    packed::stage_barrier<kPending>();
-    const Frags h0 = load(next, 0);  // past the last stage: a re-loaded copy, unused
-    __builtin_amdgcn_sched_barrier(0);
-    mfma8_dma<kSet, 0>(acc, from, cur, dma_hook(dph, ds, 0, slot, lane_off));
-    __builtin_amdgcn_sched_barrier(0);
-    cur = h0;
+    if constexpr (!kLast) step(bph, bs);
     slot = next;
   };
   // One product over all stages into set kSet, its first stage started as
-  // kStart says.
-  auto run = [&](auto setc, auto startc, Set& acc, const Set& from) __attribute__((always_inline)) {
-    stage(setc, startc, acc, from);
-    for (int s = 1; s < nstages; ++s) stage(setc, QuadC<0>{}, acc, from);
+  // kStart says. The products before an epilogue (kLast) are chained ones.
+  auto run = [&](auto setc, auto startc, auto lastc, Set& acc, const Set& from) __attribute__((always_inline)) {
+    constexpr bool kLast = decltype(lastc)::value != 0;
+    if constexpr (kLast) {
+      static_assert(decltype(startc)::value == 0, "a product before an epilogue is chained");
+      for (int s = 0; s < nstages - 1; ++s) stage(setc, startc, QuadC<0>{}, acc, from);
+      stage(setc, startc, QuadC<1>{}, acc, from);
+    } else {
+      stage(setc, startc, QuadC<0>{}, acc, from);
+      for (int s = 1; s < nstages; ++s) stage(setc, QuadC<0>{}, QuadC<0>{}, acc, from);
+    }
   };
   using SV = QuadC<kV>;
   using SA1 = QuadC<kA1>;
@@ -451,37 +454,41 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_pm(Params p) {
   using Zero = QuadC<1>;
   using From = QuadC<2>;
   using Chain = QuadC<0>;
+  using On = QuadC<0>;
+  using Last = QuadC<1>;
 
   // P5 -> V, parked as q1.
-  run(SV{}, Zero{}, V, V);
+  run(SV{}, Zero{}, On{}, V, V);
   drain<kV>(V);
   park_store<0, false>(park, wave, V, V);
   // The parked stores leave the VMEM count before the next barrier counts
   // refills again.
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   // P3 chained into V: V = C1.
-  run(SV{}, Chain{}, V, V);
+  run(SV{}, Chain{}, On{}, V, V);
   drain<kV>(V);
   // P4 -> A1.
-  run(SA1{}, Zero{}, A1, A1);
+  run(SA1{}, Zero{}, On{}, A1, A1);
   // P1 -> A2 from A1: A2 = P1 + P4; q3 = A2 + V parked.
-  run(SA2{}, From{}, A2, A1);
+  run(SA2{}, From{}, On{}, A2, A1);
   drain<kA2>(A2);
   park_store<1, true>(park, wave, A2, V);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   // P7 chained into A2: row half 0, C0 = A2 - q1, C1 = V.
-  run(SA2{}, Chain{}, A2, A2);
+  run(SA2{}, Chain{}, Last{}, A2, A2);
   drain<kA2>(A2);
   emit_half<kEpi, 1>(p, o, wave, 0, park, [&](int i, int j, const f32x16 (&pk)[1], f32x16& left, f32x16& right)
                                               __attribute__((always_inline)) {
     left = A2[i][j] - pk[0];
     right = V[i][j];
   }, tile);
+  load_stage_b();
+  cur = read_a(slot, 0);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   // P6 -> A2.
-  run(SA2{}, Zero{}, A2, A2);
+  run(SA2{}, Zero{}, On{}, A2, A2);
   // P2 chained into A1: row half 1, C2 = A1, C3 = q3 + A2 - q1 - A1.
-  run(SA1{}, Chain{}, A1, A1);
+  run(SA1{}, Chain{}, Last{}, A1, A1);
   drain<kA1>(A1);
   drain<kA2>(A2);
   emit_half<kEpi, 2>(p, o, wave, 1, park, [&](int i, int j, const f32x16 (&pk)[2], f32x16& left, f32x16& right)

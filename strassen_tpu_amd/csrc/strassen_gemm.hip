@@ -523,7 +523,7 @@ bool pm_eligible(const Params& p, const smx_gemm_desc& d) {
   if (!(d.flags & (SMX_FLAG_PRODUCT_MAJOR | SMX_FLAG_PRODUCT_MAJOR_ROUNDS))) return false;
   if (d.algo != SMX_ALGO_STRASSEN || d.b_layout != SMX_B_PACKED || p.partial) return false;
   if (p.formula != SMX_FORMULA_CLASSICAL || (p.bm / 2) % pm::TM || (p.bn / 2) % pm::TN) return false;
-  if ((p.k / 32) % pm::kQuarters) return false;  // whole pipeline stages of 64 product-space k
+  if ((p.k / 32) % pm::kMinSteps) return false;  // whole pipeline stages
   return d.epilogue == SMX_EPI_NONE || d.epilogue == SMX_EPI_SWIGLU || d.epilogue == SMX_EPI_GEGLU ||
          d.epilogue == SMX_EPI_RESIDUAL_ADD || d.epilogue == SMX_EPI_BIAS_ADD;
 }

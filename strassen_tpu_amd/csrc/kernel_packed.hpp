@@ -88,6 +88,27 @@ __device__ __forceinline__ void mfma_agpr(f32x16& c, const bf16x8& a, const bf16
 __device__ __forceinline__ void mfma_vgpr(f32x16& c, const bf16x8& a, const bf16x8& b) {
   asm("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b));
 }
+// v_mfma_f32_16x16x32_bf16, likewise. At the chip's power limit an MFMA loop
+// on random operands reaches 2.07 PFLOP/s in this shape and 1.74 to 1.82 in
+// the 32 x 32 x 16 one (whose accumulator is read and written twice as often
+// per operation). Lane l holds row (column for B) l % 16 and depth
+// 8 (l / 16) .. + 7 of an operand, and column l % 16, rows 4 (l / 16) .. + 3 of
+// the result.
+__device__ __forceinline__ void mfma16_agpr(f32x4& c, const bf16x8& a, const bf16x8& b) {
+  asm("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
+}
+__device__ __forceinline__ void mfma16_vgpr(f32x4& c, const bf16x8& a, const bf16x8& b) {
+  asm("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b));
+}
+
+// A 16 x 32 operand of that MFMA takes 16 rows of two consecutive packed
+// stages: lane l's 16 bytes are row l % 16, depth half (l / 16) % 2 of stage
+// l / 32. Byte offset of lane l from the first stage's fragment, for stages
+// `stride` bytes apart (rows 16 .. 31 of the fragment: 256 further).
+__device__ __forceinline__ uint32_t half_frag_lane(uint32_t lane, uint32_t stride) {
+  return (lane >> 5) * stride + ((lane & 15) + 32 * ((lane >> 4) & 1)) * 16;
+}
+
 // Wait states between the last MFMA writes and VALU / v_accvgpr_read reads
 // of the accumulators (more than the longest MFMA result latency). Each
 // accumulator then passes through an empty volatile asm that "defines" it,

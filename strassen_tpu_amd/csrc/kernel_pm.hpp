@@ -87,20 +87,21 @@ struct Ring {
   static constexpr int kPending = 3 * kQ;
   static_assert(kSlots >= 4 && kPending < 64, "ring depth and vmcnt range");
 };
-// Epilogue staging tile of a wave: 32 x 32 floats, rows unpadded (the ring
-// leaves 16 KB of the LDS). Same interface as StageTile.
+// Epilogue staging tile of a wave: 32 x 32 floats, each row padded by 16 bytes
+// so that the four row groups of an accumulator store (4 rows apart) fall 16
+// banks apart. Element e of the 16 x 16 block (i, j) of it, lane part excluded.
 struct Tile {
   static constexpr int kRows = 32, kCols = 32;
-  static constexpr int kStride = kCols * 4;
+  static constexpr int kStride = kCols * 4 + 16;
   static constexpr int kBytes = kRows * kStride;
-  static constexpr int at(int i, int j, int r) { return (i * 32 + 8 * (r >> 2) + (r & 3)) * kStride + j * 128; }
-  static __device__ __forceinline__ int lane_part(int lane) { return (lane >> 5) * 4 * kStride + (lane & 31) * 4; }
+  static constexpr int at(int i, int j, int e) { return (i * 16 + e) * kStride + j * 64; }
+  static __device__ __forceinline__ int lane_part(int lane) { return (lane >> 4) * 4 * kStride + (lane & 15) * 4; }
 };
 constexpr int kLds = kRingBytes + 4 * Tile::kBytes;
 static_assert(kLds <= 160 * 1024, "LDS budget");
 // One parked set of one workgroup (FP32, 128 x 256), in the registers' lane
-// order: [wave][block][4 register groups][64 lanes][4 floats]; a workgroup
-// parks two.
+// order: [wave][32 blocks of 16 x 16][64 lanes][4 floats]; a workgroup parks
+// two.
 constexpr int64_t kParkSet = (int64_t)TM * TN * 4;
 constexpr int64_t kParkBytes = 2 * kParkSet;
 
@@ -109,12 +110,13 @@ constexpr int64_t kParkBytes = 2 * kParkSet;
 constexpr uint32_t kOrder = 4u | 2u << 4 | 3u << 8 | 0u << 12 | 6u << 16 | 5u << 20 | 1u << 24;
 __host__ __device__ constexpr int product_of(int ph) { return (int)((kOrder >> (4 * ph)) & 15u); }
 
-// A wave's accumulators of one set: 128 rows x 64 columns.
-constexpr int kRowBlocks = 4, kColBlocks = 2;
-typedef f32x16 Set[kRowBlocks][kColBlocks];
+// A wave's accumulators of one set, 128 rows x 64 columns in 16 x 16 blocks,
+// and the operands of half a step: 64 rows and 64 columns of 32 k.
+constexpr int kRowBlocks = 8, kColBlocks = 4;
+typedef f32x4 Set[kRowBlocks][kColBlocks];
 
 struct FragsA {
-  bf16x8 v[kRowBlocks];
+  bf16x8 v[kRowBlocks / 2];
 };
 struct FragsB {
   bf16x8 v[kColBlocks];
@@ -124,34 +126,35 @@ struct FragsB {
 constexpr int kV = 0, kA1 = 1, kA2 = 2;
 __host__ __device__ constexpr bool in_agprs(int set) { return set != kV; }
 
-// The MFMAs of one 16-k step on a set's 4 x 2 blocks, column by column, with
-// hook(k) after MFMA k (k = 0..7) between scheduling barriers. kStart 0:
+// The MFMAs of one 32-k step on row half kHalf of a set, column by column,
+// with hook(k) after MFMA k (k = 0..15) between scheduling barriers. kStart 0:
 // chain (D = A B + D); 1: the product's first step from zero (D = A B); 2:
 // its first step from set `from` of the same file (D = A B + from).
-template <int kSet, int kStart, class Hook>
-__device__ __forceinline__ void mfma8(Set& acc, const Set& from, const FragsA& a, const FragsB& b, Hook hook) {
+template <int kSet, int kStart, int kHalf, class Hook>
+__device__ __forceinline__ void mfma16(Set& acc, const Set& from, const FragsA& a, const FragsB& b, Hook hook) {
 #pragma unroll
   for (int j = 0; j < kColBlocks; ++j)
 #pragma unroll
-    for (int i = 0; i < kRowBlocks; ++i) {
+    for (int x = 0; x < kRowBlocks / 2; ++x) {
+      const int i = kHalf * (kRowBlocks / 2) + x;
       if constexpr (kStart == 0) {
         if constexpr (in_agprs(kSet))
-          packed::mfma_agpr(acc[i][j], a.v[i], b.v[j]);
+          packed::mfma16_agpr(acc[i][j], a.v[x], b.v[j]);
         else
-          packed::mfma_vgpr(acc[i][j], a.v[i], b.v[j]);
+          packed::mfma16_vgpr(acc[i][j], a.v[x], b.v[j]);
       } else if constexpr (kStart == 1) {
         if constexpr (in_agprs(kSet))
-          asm("v_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=&a"(acc[i][j]) : "v"(a.v[i]), "v"(b.v[j]));
+          asm("v_mfma_f32_16x16x32_bf16 %0, %1, %2, 0" : "=&a"(acc[i][j]) : "v"(a.v[x]), "v"(b.v[j]));
         else
-          asm("v_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=&v"(acc[i][j]) : "v"(a.v[i]), "v"(b.v[j]));
+          asm("v_mfma_f32_16x16x32_bf16 %0, %1, %2, 0" : "=&v"(acc[i][j]) : "v"(a.v[x]), "v"(b.v[j]));
       } else {
         static_assert(in_agprs(kSet), "only the AGPR sets start from another set");
-        asm("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %3"
+        asm("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %3"
             : "=&a"(acc[i][j])
-            : "v"(a.v[i]), "v"(b.v[j]), "a"(from[i][j]));
+            : "v"(a.v[x]), "v"(b.v[j]), "a"(from[i][j]));
       }
       __builtin_amdgcn_sched_barrier(0);
-      hook(kRowBlocks * j + i);
+      hook((kRowBlocks / 2) * j + x);
       __builtin_amdgcn_sched_barrier(0);
     }
 }
@@ -178,10 +181,10 @@ __device__ __forceinline__ void drain(Set& acc) {
 // Parked sets go through a buffer resource over the workgroup's park
 // region: a uniform base, the lane's 32-bit byte offset (derived where it is
 // used, so no per-lane 64-bit address is held across the main loops) and a
-// compile-time offset. Lane l of register group g of block (i, j) of set x
-// of wave w sits at x kParkSet + w kParkSet / 4 + (4 (2 i + j) + g) KB + 16 l.
-__device__ __forceinline__ uint32_t park_offset(int set, int wave, int i, int j, int g) {
-  return (uint32_t)(set * kParkSet + wave * (kParkSet / 4) + ((kColBlocks * i + j) * 4 + g) * 1024);
+// compile-time offset. Lane l of the 16 x 16 block (i, j) of set x of wave w sits
+// at x kParkSet + w kParkSet / 4 + (4 i + j) KB + 16 l.
+__device__ __forceinline__ uint32_t park_offset(int set, int wave, int i, int j) {
+  return (uint32_t)(set * kParkSet + wave * (kParkSet / 4) + (kColBlocks * i + j) * 1024);
 }
 
 // Stores x (plus y, when kAdd) as parked set kSetIdx.
@@ -191,29 +194,30 @@ __device__ __forceinline__ void park_store(__amdgpu_buffer_rsrc_t park, int wave
 #pragma unroll
   for (int i = 0; i < kRowBlocks; ++i)
 #pragma unroll
-    for (int j = 0; j < kColBlocks; ++j)
+    for (int j = 0; j < kColBlocks; ++j) {
+      f32x4 v;
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        f32x4 v;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = kAdd ? x[i][j][4 * g + e] + y[i][j][4 * g + e] : x[i][j][4 * g + e];
-        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), park, lane16,
-                                               park_offset(kSetIdx, wave, i, j, g), 0);
-      }
+      for (int e = 0; e < 4; ++e) v[e] = kAdd ? x[i][j][e] + y[i][j][e] : x[i][j][e];
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), park, lane16,
+                                             park_offset(kSetIdx, wave, i, j), 0);
+    }
 }
 
-// Block (i, j) of parked set kSetIdx.
+// 32 x 32 block (bi, bj) of parked set kSetIdx, as 2 x 2 blocks.
+struct Block {
+  f32x4 v[2][2];
+};
 template <int kSetIdx>
-__device__ __forceinline__ f32x16 park_block(__amdgpu_buffer_rsrc_t park, int wave, uint32_t lane16, int i, int j) {
-  f32x16 v;
+__device__ __forceinline__ Block park_block(__amdgpu_buffer_rsrc_t park, int wave, uint32_t lane16, int bi, int bj) {
+  Block r;
 #pragma unroll
-  for (int g = 0; g < 4; ++g) {
-    const f32x4 x = __builtin_bit_cast(
-        f32x4, __builtin_amdgcn_raw_buffer_load_b128(park, lane16, park_offset(kSetIdx, wave, i, j, g), 0));
+  for (int i = 0; i < 2; ++i)
 #pragma unroll
-    for (int e = 0; e < 4; ++e) v[4 * g + e] = x[e];
-  }
-  return v;
+    for (int j = 0; j < 2; ++j)
+      r.v[i][j] = __builtin_bit_cast(
+          f32x4, __builtin_amdgcn_raw_buffer_load_b128(park, lane16,
+                                                       park_offset(kSetIdx, wave, 2 * bi + i, 2 * bj + j), 0));
+  return r;
 }
 
 // Parked blocks are loaded this many blocks ahead of their use: the parks
@@ -222,55 +226,62 @@ __device__ __forceinline__ f32x16 park_block(__amdgpu_buffer_rsrc_t park, int wa
 // more, and more spill.
 constexpr int kParkAhead = 2;
 
-// Epilogue of logical row half lr. quads(i, j, pk, left, right) yields
-// the FP32 values of quadrants (lr, 0) and (lr, 1) of the wave's block
-// (i, j), given block (i, j) of parked sets 0 .. kParks-1 (pk[0], pk[1]),
-// loaded kParkAhead blocks ahead. One 32 x 32 block at a
-// time passes through the wave's staging tile (strassen_pallas.py:739-792,
-// :867-874): SwiGLU / GeGLU store gate(left) * right into [M, N/2];
-// residual_add and bias_add (and no epilogue) store each quadrant. Logical
-// quadrant (row, col) is stored at physical (row ^ swap_m, col ^ swap_n)
-// for the block permutation (strassen_pallas.py:205-226).
+// Epilogue of logical row half lr. quads(i, j, q1, q3, left, right) yields the
+// FP32 values of quadrants (lr, 0) and (lr, 1) of the wave's 16 x 16 block
+// (i, j), given that block of the parked sets (q3 only when kParks is 2),
+// loaded kParkAhead 32 x 32 blocks ahead. One 32 x 32 block at a time passes
+// through the wave's staging tile (strassen_pallas.py:739-792, :867-874):
+// SwiGLU / GeGLU store gate(left) * right into [M, N/2]; residual_add and
+// bias_add (and no epilogue) store each quadrant. Logical quadrant (row, col)
+// is stored at physical (row ^ swap_m, col ^ swap_n) for the block
+// permutation (strassen_pallas.py:205-226).
 template <int kEpi, int kParks, class Quads>
 __device__ __forceinline__ void emit_half(const Params& p, const TileOrigin& o, int wave, int lr,
                                           __amdgpu_buffer_rsrc_t park, Quads quads, uint8_t* tile) {
   using T = Tile;
+  constexpr int kBlocksM = kRowBlocks / 2, kBlocksN = kColBlocks / 2, kCount = kBlocksM * kBlocksN;
   const int lane = opaque_lane_id();
-  const int lcol = lane & 31;
   const int64_t hm = p.bm / 2, hn = p.bn / 2;
   const int swap_m = p.perm & 1, swap_n = (p.perm >> 2) & 1;
   const int64_t half = lr ^ swap_m;
   const int es = p.out_f32 ? 4 : 2;
   uint8_t* const te = tile + T::lane_part(lane);
   auto fence = []() __attribute__((always_inline)) { asm volatile("" ::: "memory"); };
-  auto put = [&](int r, float v) __attribute__((always_inline)) {
-    *reinterpret_cast<float*>(te + T::at(0, 0, r)) = v;
-  };
-  auto get = [&](int r) __attribute__((always_inline)) {
-    return *reinterpret_cast<const float*>(te + T::at(0, 0, r));
+  auto at = [&](int i, int j, int e) __attribute__((always_inline)) {
+    return reinterpret_cast<float*>(te + T::at(i, j, e));
   };
   const uint32_t lane16 = lane * 16;
-  f32x16 pk[kParkAhead + 1][kParks];
-  auto fetch = [&](f32x16 (&to)[kParks], int b) __attribute__((always_inline)) {
-    to[0] = park_block<0>(park, wave, lane16, b / kColBlocks, b % kColBlocks);
-    if constexpr (kParks > 1) to[kParks - 1] = park_block<kParks - 1>(park, wave, lane16, b / kColBlocks, b % kColBlocks);
+  Block pk[kParkAhead + 1][kParks];
+  auto fetch = [&](Block (&to)[kParks], int b) __attribute__((always_inline)) {
+    to[0] = park_block<0>(park, wave, lane16, b / kBlocksN, b % kBlocksN);
+    if constexpr (kParks > 1) to[kParks - 1] = park_block<kParks - 1>(park, wave, lane16, b / kBlocksN, b % kBlocksN);
   };
 #pragma unroll
   for (int f = 0; f < kParkAhead; ++f) fetch(pk[f], f);
 #pragma unroll
-  for (int b = 0; b < 8; ++b) {
-    const int i = b / kColBlocks, j = b % kColBlocks;
-    if (b + kParkAhead < 8) fetch(pk[(b + kParkAhead) % (kParkAhead + 1)], b + kParkAhead);
-    const int64_t row = o.ti * p.bm + o.tr + i * 32 + half * hm;
-    const int64_t cc = o.tc + wave * 64 + j * 32;  // column inside a column half
-    f32x16 left, right;
-    quads(i, j, pk[b % (kParkAhead + 1)], left, right);
+  for (int b = 0; b < kCount; ++b) {
+    const int bi = b / kBlocksN, bj = b % kBlocksN;
+    if (b + kParkAhead < kCount) fetch(pk[(b + kParkAhead) % (kParkAhead + 1)], b + kParkAhead);
+    const Block(&q)[kParks] = pk[b % (kParkAhead + 1)];
+    const int64_t row = o.ti * p.bm + o.tr + bi * 32 + half * hm;
+    const int64_t cc = o.tc + wave * 64 + bj * 32;  // column inside a column half
+    Block left, right;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        quads(2 * bi + i, 2 * bj + j, q[0].v[i][j], q[kParks - 1].v[i][j], left.v[i][j], right.v[i][j]);
     if constexpr (kEpi == SMX_EPI_SWIGLU || kEpi == SMX_EPI_GEGLU) {
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const float gate = swap_n ? right[r] : left[r], up = swap_n ? left[r] : right[r];
-        put(r, gate_f32<kEpi>(gate) * up);
-      }
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const float gate = swap_n ? right.v[i][j][e] : left.v[i][j][e];
+            const float up = swap_n ? left.v[i][j][e] : right.v[i][j][e];
+            *at(i, j, e) = gate_f32<kEpi>(gate) * up;
+          }
       fence();
       tile_store<T>(tile, reinterpret_cast<char*>(p.c) + (row * p.ldc + o.tj * hn + cc) * es, p.ldc, p.out_f32,
                     lane);
@@ -285,14 +296,19 @@ __device__ __forceinline__ void emit_half(const Params& p, const TileOrigin& o, 
                        p.residual_f32, lane);
           fence();
         }
-        float bv = 0.f;
-        if constexpr (kEpi == SMX_EPI_BIAS_ADD) bv = load_vec(p.bias, p.bias_f32, col + lcol);
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          float v = lc ? right[r] : left[r];
-          if constexpr (kEpi == SMX_EPI_RESIDUAL_ADD) v += get(r);
-          if constexpr (kEpi == SMX_EPI_BIAS_ADD) v += bv;
-          put(r, v);
+        for (int j = 0; j < 2; ++j) {
+          float bv = 0.f;
+          if constexpr (kEpi == SMX_EPI_BIAS_ADD) bv = load_vec(p.bias, p.bias_f32, col + j * 16 + (lane & 15));
+#pragma unroll
+          for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              float v = lc ? right.v[i][j][e] : left.v[i][j][e];
+              if constexpr (kEpi == SMX_EPI_RESIDUAL_ADD) v += *at(i, j, e);
+              if constexpr (kEpi == SMX_EPI_BIAS_ADD) v += bv;
+              *at(i, j, e) = v;
+            }
         }
         fence();
         tile_store<T>(tile, reinterpret_cast<char*>(p.c) + (row * p.ldc + col) * es, p.ldc, p.out_f32, lane);
@@ -323,7 +339,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_pm(Params p) {
   const uint32_t panel = (uint32_t)nst16 * kPackedStage;
   const __amdgpu_buffer_rsrc_t a_src = packed::panel_rsrc(
       reinterpret_cast<const uint8_t*>(p.a) + (int64_t)tile_m * panel + wave * kFrag, panel - wave * kFrag);
-  const uint32_t b_block = (wave & 1) * kColBlocks * kFrag;
+  const uint32_t b_block = (wave & 1) * 2 * kFrag;
   const __amdgpu_buffer_rsrc_t b_src = packed::panel_rsrc(
       reinterpret_cast<const uint8_t*>(p.b) + (int64_t)(2 * tile_n + (wave >> 1)) * panel + b_block, panel - b_block);
   // The workgroup's parked sets q1 and q3.
@@ -331,47 +347,59 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_pm(Params p) {
       reinterpret_cast<const uint8_t*>(p.park) + (int64_t)blockIdx.x * kParkBytes, (uint32_t)kParkBytes);
   uint8_t* const tile = lds + kRingBytes + wave * Tile::kBytes;
 
-  // Byte offset of step q of stage (ph, s) in a panel. Stages past the last
-  // one re-load it (in bounds, never used).
-  auto step_offset = [&](int ph, int s, int q) __attribute__((always_inline)) {
-    if (ph >= kOps) {
-      ph = kOps - 1;
-      s = nstages - 1;
-    }
-    return (uint32_t)((kQ * s + q) * kOps + product_of(ph)) * kOpStage;
+  // A stream of stages through the products: `at` is the byte offset of the
+  // current stage's first step in a panel. Kept incrementally, so that a VMEM
+  // operation between two MFMAs costs one scalar addition and not the
+  // address of its step: the wave's other instructions only issue for free in
+  // the 12 cycles that an MFMA leaves. Past the last stage it stays there
+  // (in bounds, loaded again and never used).
+  constexpr uint32_t kStageStep = kQ * kPackedStage;  // to the product's next stage
+  struct Stream {
+    int ph = 0, s = 0;
+    uint32_t at = product_of(0) * kOpStage;
   };
-  auto dma_a = [&](int ph, int s, int q, int slot, uint32_t lane16) __attribute__((always_inline)) {
-    packed::dma_frag(a_src, lane16, step_offset(ph, s, q), lds + slot * R::kStageBytes + q * kOpStage + wave * kFrag);
+  auto advance = [&](Stream& x) __attribute__((always_inline)) {
+    // selects, not branches: the loop stays one block
+    const int s1 = x.s + 1;
+    const bool wraps = s1 == nstages, ends = x.ph == kOps - 1;
+    const int ph = wraps && !ends ? x.ph + 1 : x.ph;
+    x.at = wraps ? (ends ? x.at : (uint32_t)product_of(ph) * kOpStage) : x.at + kStageStep;
+    x.s = wraps ? (ends ? x.s : 0) : s1;
+    x.ph = ph;
   };
-  auto load_b = [&](int ph, int s, int q, int j, uint32_t lane16) __attribute__((always_inline)) {
+  auto dma_a = [&](uint32_t at, int q, int slot, uint32_t lane16) __attribute__((always_inline)) {
+    packed::dma_frag(a_src, lane16, at + q * kPackedStage, lds + slot * R::kStageBytes + q * kOpStage + wave * kFrag);
+  };
+  // Columns 16 j .. of the wave's 64 in 32-k step t of the stage at `at`, and
+  // rows 64 h + 16 x .. of A's step q / 2, h = q % 2.
+  auto load_b = [&](uint32_t at, int t, int j, uint32_t lane_b) __attribute__((always_inline)) {
     return __builtin_bit_cast(
-        bf16x8, __builtin_amdgcn_raw_buffer_load_b128(b_src, lane16 + j * kFrag, step_offset(ph, s, q), 0));
+        bf16x8, __builtin_amdgcn_raw_buffer_load_b128(b_src, lane_b + (j >> 1) * kFrag + (j & 1) * (kFrag / 4),
+                                                      at + 2 * t * kPackedStage, 0));
   };
-  auto read_a = [&](int slot, int q) __attribute__((always_inline)) {
-    const uint8_t* const base = lds + slot * R::kStageBytes + q * kOpStage + opaque_lane_id() * 16;
+  auto a_base = [&](int slot, uint32_t lane) __attribute__((always_inline)) {
+    return lds + slot * R::kStageBytes + packed::half_frag_lane(lane, kOpStage);
+  };
+  auto read_a = [&](const uint8_t* base, int q, int x) __attribute__((always_inline)) {
+    return packed::ld_frag(base + (q & ~1) * kOpStage + (q & 1) * 2 * kFrag + (x >> 1) * kFrag +
+                           (x & 1) * (kFrag / 4));
+  };
+  auto read_a_half = [&](const uint8_t* base, int q) __attribute__((always_inline)) {
     FragsA f;
 #pragma unroll
-    for (int i = 0; i < kRowBlocks; ++i) f.v[i] = packed::ld_frag(base + i * kFrag);
+    for (int x = 0; x < kRowBlocks / 2; ++x) f.v[x] = read_a(base, q, x);
     return f;
   };
 
-  // Stage counters of the A refill (dph, ds) and of the B loads (bph, bs),
-  // stepped through the products' stages.
-  auto step = [&](int& ph, int& s) __attribute__((always_inline)) {
-    if (++s == nstages) {
-      s = 0;
-      ++ph;
-    }
-  };
-  int dph = 0, ds = 0, bph = 0, bs = 0;
-  FragsB b[kQ];
+  Stream da, db;  // A's refill, B's loads
+  FragsB b[kQ / 2];
   auto load_stage_b = [&]() __attribute__((always_inline)) {
-    const uint32_t lane16 = opaque_lane_id() * 16;
+    const uint32_t lane_b = packed::half_frag_lane(opaque_lane_id(), kPackedStage);
 #pragma unroll
-    for (int q = 0; q < kQ; ++q)
+    for (int t = 0; t < kQ / 2; ++t)
 #pragma unroll
-      for (int j = 0; j < kColBlocks; ++j) b[q].v[j] = load_b(bph, bs, q, j, lane16);
-    step(bph, bs);
+      for (int j = 0; j < kColBlocks; ++j) b[t].v[j] = load_b(db.at, t, j, lane_b);
+    advance(db);
   };
   // Prologue: A's stage 0, B's stage 0, A's stages 1 .. kSlots - 2, and the
   // first step of the refill that the stage loop goes on with.
@@ -380,59 +408,76 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_pm(Params p) {
 #pragma unroll
     for (int st = 0; st < R::kSlots - 1; ++st) {
 #pragma unroll
-      for (int q = 0; q < kQ; ++q) dma_a(dph, ds, q, st, lane16);
-      step(dph, ds);
+      for (int q = 0; q < kQ; ++q) dma_a(da.at, q, st, lane16);
+      advance(da);
       if (st == 0) load_stage_b();
     }
-    dma_a(dph, ds, 0, R::kSlots - 1, lane16);
+    dma_a(da.at, 0, R::kSlots - 1, lane16);
   }
   packed::stage_barrier<0>();
 
   Set V, A1, A2;
   int slot = 0;
-  FragsA cur = read_a(0, 0);
+  FragsA cur = read_a_half(a_base(0, opaque_lane_id()), 0);
 
-  // One pipeline stage: each step's A fragments read under the previous
-  // step's MFMAs; behind each step's MFMAs one A DMA of the refill of the
-  // slot read at the previous stage (its steps 1 .. kQ - 1 during the first
-  // kQ - 1 steps) and the step's B fragments of the next stage, one VMEM
-  // operation at a time between two MFMAs. Before the last step the barrier:
-  // every wave has then read all of this stage's slot, whose refill starts
-  // behind it, and A's next stage has landed. kStart applies to the first
-  // step (the product's first stage). kLast: an epilogue follows, which
-  // needs the registers: nothing is loaded ahead.
+  // One pipeline stage of kQ half steps (32 k of 64 rows each): every half's A
+  // fragments are read under the half before; behind its MFMAs goes one A DMA
+  // of the refill of the slot read at the previous stage (its 16-k steps 1 ..
+  // kQ - 1 during the first kQ - 1 halves) and, in a step's second half, as each
+  // column's last MFMA has gone, its B fragment of the next stage. Before the
+  // last half the barrier: every wave has then read all of this stage's
+  // slot, whose refill starts behind it, and A's next stage has landed. kStart
+  // applies to the first step (the product's first stage). kLast: an epilogue
+  // follows, which needs the registers: nothing is loaded ahead.
   auto stage = [&](auto setc, auto startc, auto lastc, Set& acc, const Set& from) __attribute__((always_inline)) {
     constexpr int kSet = decltype(setc)::value, kStart = decltype(startc)::value;
     constexpr bool kLast = decltype(lastc)::value != 0;
     const int next = slot == R::kSlots - 1 ? 0 : slot + 1;
     const int fill = slot == 0 ? R::kSlots - 1 : slot - 1;
-    const uint32_t lane16 = opaque_lane_id() * 16;
+    const uint32_t lane = opaque_lane_id();
+    const uint32_t lane16 = lane * 16, lane_b = packed::half_frag_lane(lane, kPackedStage);
+    const uint8_t* const base = a_base(slot, lane);
+    const uint8_t* const next_base = a_base(next, lane);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int q = 0; q < kQ; ++q) {
       FragsA nxt{};
-      if (q < kQ - 1) {
-        nxt = read_a(slot, q + 1);
-      } else {
-        step(dph, ds);
-        packed::stage_barrier<R::kPending>();
-        if constexpr (!kLast) nxt = read_a(next, 0);  // past the last stage: a re-loaded copy, unused
-      }
+      // One wait per half for its fragments, in place of one per fragment: A's
+      // were read under the last half; a step's B loads have all but the
+      // newest stage's operations less its own six behind them (fewer before
+      // an epilogue, where the compiler adds what is missing).
+      if (q % 2 == 0)
+        __builtin_amdgcn_s_waitcnt(packed::waitcnt_imm(3 * kQ - 6, 0));
+      else
+        __builtin_amdgcn_s_waitcnt(packed::waitcnt_imm(63, 0));
+      if (q == kQ - 1) packed::stage_barrier<R::kPending>();
       __builtin_amdgcn_sched_barrier(0);
+      FragsB& bt = b[q / 2];
       auto hook = [&](int k) __attribute__((always_inline)) {
-        if (k == 1) dma_a(dph, ds, q < kQ - 1 ? q + 1 : 0, q < kQ - 1 ? fill : slot, lane16);
-        if constexpr (!kLast) {
-          if (k == 4) b[q].v[0] = load_b(bph, bs, q, 0, lane16);
-          if (k == 7) b[q].v[1] = load_b(bph, bs, q, 1, lane16);
+        if (k == 1) dma_a(da.at, q < kQ - 1 ? q + 1 : 0, q < kQ - 1 ? fill : slot, lane16);
+        if (k >= 4 && k % 2 == 0 && k < 12) {
+          const int x = (k - 4) / 2;
+          if (q < kQ - 1)
+            nxt.v[x] = read_a(base, q + 1, x);
+          else if (!kLast)
+            nxt.v[x] = read_a(next_base, 0, x);  // past the last stage: a re-loaded copy, unused
         }
+        if constexpr (!kLast) {
+          if (q % 2 == 1 && k % 4 == 3) bt.v[k / 4] = load_b(db.at, q / 2, k / 4, lane_b);
+          if (q == kQ - 1 && k == 15) advance(db);
+        }
+        if (q == kQ - 2 && k == 14) advance(da);
       };
       if (q == 0)
-        mfma8<kSet, kStart>(acc, from, cur, b[q], hook);
+        mfma16<kSet, kStart, 0>(acc, from, cur, bt, hook);
+      else if (q == 1)
+        mfma16<kSet, kStart, 1>(acc, from, cur, bt, hook);
+      else if (q % 2 == 0)
+        mfma16<kSet, 0, 0>(acc, from, cur, bt, hook);
       else
-        mfma8<kSet, 0>(acc, from, cur, b[q], hook);
+        mfma16<kSet, 0, 1>(acc, from, cur, bt, hook);
       cur = nxt;
     }
-    if constexpr (!kLast) step(bph, bs);
     slot = next;
   };
   // One product over all stages into set kSet, its first stage started as
@@ -477,13 +522,13 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_pm(Params p) {
   // P7 chained into A2: row half 0, C0 = A2 - q1, C1 = V.
   run(SA2{}, Chain{}, Last{}, A2, A2);
   drain<kA2>(A2);
-  emit_half<kEpi, 1>(p, o, wave, 0, park, [&](int i, int j, const f32x16 (&pk)[1], f32x16& left, f32x16& right)
+  emit_half<kEpi, 1>(p, o, wave, 0, park, [&](int i, int j, const f32x4& q1, const f32x4&, f32x4& left, f32x4& right)
                                               __attribute__((always_inline)) {
-    left = A2[i][j] - pk[0];
+    left = A2[i][j] - q1;
     right = V[i][j];
   }, tile);
   load_stage_b();
-  cur = read_a(slot, 0);
+  cur = read_a_half(a_base(slot, opaque_lane_id()), 0);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   // P6 -> A2.
   run(SA2{}, Zero{}, On{}, A2, A2);
@@ -491,10 +536,10 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_pm(Params p) {
   run(SA1{}, Chain{}, Last{}, A1, A1);
   drain<kA1>(A1);
   drain<kA2>(A2);
-  emit_half<kEpi, 2>(p, o, wave, 1, park, [&](int i, int j, const f32x16 (&pk)[2], f32x16& left, f32x16& right)
+  emit_half<kEpi, 2>(p, o, wave, 1, park, [&](int i, int j, const f32x4& q1, const f32x4& q3, f32x4& left, f32x4& right)
                                               __attribute__((always_inline)) {
     left = A1[i][j];
-    right = ((pk[1] + A2[i][j]) - pk[0]) - A1[i][j];
+    right = ((q3 + A2[i][j]) - q1) - A1[i][j];
   }, tile);
   // Every wave's DMA (the unread re-loads past the last stage) has landed
   // before the workgroup ends.

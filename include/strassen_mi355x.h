@@ -326,6 +326,16 @@ int smx_norm_residual_add(int64_t m, int64_t n, const float* x, int64_t ldx, con
                           const void* scale, int32_t dtypes, float eps, void* out, int64_t ldo, void* stream);
 
 /*
+ * RMSNorm of bf16 rows (the decoder layer's rms_norm,
+ * experiments/qwen3/benchmark_qwen3_32b_layer.py:270-276): out = x *
+ * rsqrt(mean_row(x^2) + eps) * scale in FP32, rounded once to bf16, x and out
+ * bf16 [m, n], scale [n] bf16 or float32 (SMX_NRA_SCALE_F32). Needs n % 8 == 0
+ * and 16-byte aligned rows and scale. Asynchronous on stream.
+ */
+int smx_rms_norm(int64_t m, int64_t n, const void* x, int64_t ldx, const void* scale, int32_t dtypes, float eps,
+                 void* out, int64_t ldo, void* stream);
+
+/*
  * Second pass of the qk_norm_rope epilogue (strassen_pallas.py:793-835) for
  * head widths the fused epilogue does not take (it fuses head_dim 128): from
  * the FP32 product x [m, n] (an smx_gemm with SMX_FLAG_OUT_F32 and no

@@ -59,7 +59,7 @@ SMX_QK_SCALE_F32 = 1
 SMX_QK_OUT_F32 = 4
 
 EXPORTS = ("smx_gemm", "smx_gemm_noalloc", "smx_gemm_workspace_bytes", "smx_matmul", "smx_matmul_workspace_bytes",
-           "smx_tile_requirements", "smx_packed_bytes", "smx_pack_operand", "smx_pack_rhs_transposed", "smx_norm_residual_add", "smx_qk_norm_rope", "smx_last_error", "smx_version")
+           "smx_tile_requirements", "smx_packed_bytes", "smx_pack_operand", "smx_pack_rhs_transposed", "smx_norm_residual_add", "smx_rms_norm", "smx_qk_norm_rope", "smx_last_error", "smx_version")
 
 
 class SmxGemmDesc(ctypes.Structure):
@@ -118,6 +118,8 @@ def load():
     f32 = ctypes.c_float
     lib.smx_norm_residual_add.argtypes = [i64, i64, vp, i64, vp, i64, vp, i32, f32, vp, i64, vp]
     lib.smx_norm_residual_add.restype = ctypes.c_int
+    lib.smx_rms_norm.argtypes = [i64, i64, vp, i64, vp, i32, f32, vp, i64, vp]
+    lib.smx_rms_norm.restype = ctypes.c_int
     lib.smx_qk_norm_rope.argtypes = [i64, i64, vp, i64, vp, vp, vp, i32, i32, i32, f32, vp, i64, vp]
     lib.smx_qk_norm_rope.restype = ctypes.c_int
     lib.smx_last_error.argtypes = []

@@ -100,6 +100,24 @@ def rms_norm(x, scale, eps):
     return (x32 * torch.rsqrt(x32.square().mean(-1, keepdim=True) + eps) * scale.float()).to(torch.bfloat16)
 
 
+def _row_rms_norm(x, scale, eps):
+    """``rms_norm`` of a block's hidden state ``[tokens, hidden]`` in one pass
+    on the device (``smx_rms_norm``), the fused arms' norm. Its callers feed it
+    to kernels that carry no gradient. Other layouts and types take the
+    torch form."""
+    if (x.device.type != "cuda" or x.dtype != torch.bfloat16 or x.dim() != 2 or not x.is_contiguous()
+            or scale.device != x.device or scale.dtype not in (torch.bfloat16, torch.float32)
+            or not scale.is_contiguous() or tuple(scale.shape) != (x.shape[1],) or not x.numel() or x.shape[1] % 8
+            or x.data_ptr() % 16 or scale.data_ptr() % 16):
+        return rms_norm(x, scale, eps)
+    out = torch.empty_like(x)
+    stream = torch.cuda.current_stream(x.device).cuda_stream
+    _lib.check(_lib.load().smx_rms_norm(x.shape[0], x.shape[1], _lib.ptr(x), x.stride(0), _lib.ptr(scale),
+                                        _lib.SMX_NRA_SCALE_F32 if scale.dtype == torch.float32 else 0, float(eps),
+                                        _lib.ptr(out), out.stride(0), stream))
+    return out
+
+
 def apply_rope(x, cos, sin):
     """RoPE on ``[batch, seq, heads, head_dim]`` with ``[seq, head_dim]``
     tables (``:279-284``)."""
@@ -123,9 +141,22 @@ def attention(query, key, value):
     Runs on torch's fused SDPA kernels only (flash or memory-efficient); the
     math backend is excluded because its batched bf16 products on transposed
     views are not safe on this GPU, so an unsupported shape raises instead.
+
+    On the device the flash kernel reads the heads as they lie and shares
+    each key and value head among its query heads; elsewhere, with gradients
+    to record or for shapes it may not take, they are laid out head by head
+    and repeated first.
     """
     from torch.nn.attention import SDPBackend, sdpa_kernel
 
+    if (query.device.type == "cuda" and query.dtype == torch.bfloat16 and query.shape[3] == 128
+            and query.shape[2] % key.shape[2] == 0 and query.shape[1] == key.shape[1] > 0
+            and all(t.stride(3) == 1 for t in (query, key, value))
+            and not (torch.is_grad_enabled() and any(t.requires_grad for t in (query, key, value)))):
+        with sdpa_kernel([SDPBackend.FLASH_ATTENTION, SDPBackend.EFFICIENT_ATTENTION]):
+            out = torch.nn.functional.scaled_dot_product_attention(
+                query.transpose(1, 2), key.transpose(1, 2), value.transpose(1, 2), is_causal=True, enable_gqa=True)
+        return out.transpose(1, 2)
     groups = query.shape[2] // key.shape[2]
     q = query.transpose(1, 2).contiguous()
     k = key.repeat_interleave(groups, dim=2).transpose(1, 2).contiguous()
@@ -179,7 +210,8 @@ def block_forward(x, block):
     """One decoder block: ``x [batch*seq, hidden]`` bf16 -> same shape."""
     d, w = block.dims, block.weights
     batch, seq = block.batch, block.seq
-    normalized = rms_norm(x, w.attention_norm, d.eps)
+    norm = rms_norm if block.arm in ("hipblaslt", "cubic_unfused") else _row_rms_norm
+    normalized = norm(x, w.attention_norm, d.eps)
     if block.arm in ("hipblaslt", "cubic_unfused"):
         query = torch.matmul(normalized, w.query).view(batch, seq, d.heads, d.head_dim)
         key = torch.matmul(normalized, w.key).view(batch, seq, d.kv_heads, d.head_dim)
@@ -209,6 +241,6 @@ def block_forward(x, block):
         activated = (torch.nn.functional.silu(gate.float()) * up.float()).to(torch.bfloat16)
         return (residual.float() + block.gemm(activated, block.mlp_down).float()).to(torch.bfloat16)
     residual = block.gemm(attended, block.attention_output, epilogue="residual_add", residual=x)
-    normalized = rms_norm(residual, w.mlp_norm, d.eps)
+    normalized = _row_rms_norm(residual, w.mlp_norm, d.eps)
     activated = block.gemm(normalized, block.gate_up, epilogue="swiglu")
     return block.gemm(activated, block.mlp_down, epilogue="residual_add", residual=residual)

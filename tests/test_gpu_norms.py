@@ -1,0 +1,79 @@
+"""GPU row norms (smx_rms_norm, smx_norm_residual_add's chunked pass) against
+their FP32 definition, at widths below, at and past what a workgroup keeps in
+registers, and the block's attention against its head-by-head layout."""
+
+import pytest
+import torch
+
+import strassen_tpu_amd.qwen3_block as qb
+from strassen_tpu_amd import _lib
+from test_gpu_parity import DEV, say
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(autouse=True)
+def _announce(request):
+    say(f"\n[gpu] {request.node.nodeid}")
+    yield
+    torch.cuda.synchronize()
+
+
+def _ulp_close(got, want):
+    """Within one bf16 ulp: FP32 sums of n squares in another order differ by
+    under n 2^-24, far below half an ulp (2^-9)."""
+    assert ((got.double() - want).abs() <= want.abs() * 2.0 ** -7 + 1e-30).all()
+
+
+@pytest.mark.parametrize("m,n", [(1, 8), (3, 2040), (5, 5120), (2, 8192), (2, 8200), (1, 25600)])
+@pytest.mark.parametrize("scale_dtype", [torch.bfloat16, torch.float32])
+def test_rms_norm(m, n, scale_dtype):
+    g = torch.Generator(device=DEV).manual_seed(n)
+    x = (torch.randn(m, n, device=DEV, generator=g) * 3).to(torch.bfloat16)
+    scale = torch.randn(n, device=DEV, generator=g).to(scale_dtype)
+    x64 = x.double()
+    want = x64 * torch.rsqrt(x64.square().mean(-1, keepdim=True) + 1e-6) * scale.double()
+    _ulp_close(qb._row_rms_norm(x, scale, 1e-6), want)
+    _ulp_close(qb.rms_norm(x, scale, 1e-6), want)
+
+
+def test_rms_norm_keeps_other_layouts():
+    """Widths and views that are not whole 16-byte chunks take the torch form."""
+    x = torch.randn(4, 100, device=DEV).to(torch.bfloat16)
+    scale = torch.randn(100, device=DEV).to(torch.bfloat16)
+    assert torch.equal(qb._row_rms_norm(x, scale, 1e-6), qb.rms_norm(x, scale, 1e-6))
+    wide = torch.randn(4, 130, device=DEV).to(torch.bfloat16)[:, 1:129]
+    scale = torch.randn(128, device=DEV).to(torch.bfloat16)
+    assert torch.equal(qb._row_rms_norm(wide, scale, 1e-6), qb.rms_norm(wide, scale, 1e-6))
+
+
+# chunked rows, and rows that are not (odd width, odd stride)
+@pytest.mark.parametrize("m,n,pad", [(3, 256, 0), (2, 8192, 0), (2, 8448, 8), (3, 250, 0), (3, 256, 1)])
+@pytest.mark.parametrize("f32", [False, True])
+def test_norm_residual_add(m, n, pad, f32):
+    g = torch.Generator(device=DEV).manual_seed(n + pad)
+    dtype = torch.float32 if f32 else torch.bfloat16
+    x = torch.randn(m, n + pad, device=DEV, generator=g)[:, :n]
+    residual = torch.randn(m, n + pad, device=DEV, generator=g).to(dtype)[:, :n]
+    scale = torch.randn(n, device=DEV, generator=g).to(dtype)
+    out = torch.empty(m, n, device=DEV, dtype=dtype)
+    bits = _lib.SMX_NRA_SCALE_F32 | _lib.SMX_NRA_RESIDUAL_F32 | _lib.SMX_NRA_OUT_F32 if f32 else 0
+    _lib.check(_lib.load().smx_norm_residual_add(
+        m, n, x.data_ptr(), x.stride(0), residual.data_ptr(), residual.stride(0), scale.data_ptr(), bits, 1e-6,
+        out.data_ptr(), out.stride(0), torch.cuda.current_stream(DEV).cuda_stream))
+    x64 = x.double()
+    product = x64 * torch.rsqrt(x64.square().mean(-1, keepdim=True) + 1e-6) * scale.double()
+    want = product + residual.double()
+    # one rounding of the result, FP32 rounding of its terms
+    eps = 2.0 ** -23 if f32 else 2.0 ** -8
+    bound = want.abs() * eps + (product.abs() + residual.double().abs()) * 2.0 ** -20
+    assert ((out.double() - want).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("heads,kv", [(8, 8), (16, 2)])
+def test_attention_reads_heads_in_place(heads, kv):
+    g = torch.Generator(device=DEV).manual_seed(1)
+    q, k, v = (torch.randn(2, 256, h, 128, device=DEV, generator=g).to(torch.bfloat16) for h in (heads, kv, kv))
+    with torch.enable_grad():
+        want = qb.attention(q.detach().requires_grad_(), k, v).detach()  # laid out and repeated
+    assert torch.equal(qb.attention(q, k, v), want)

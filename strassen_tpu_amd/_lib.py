@@ -9,6 +9,7 @@ one HIP context and torch's streams are valid handles here.
 from __future__ import annotations
 
 import ctypes
+import functools
 import os
 
 import torch  # noqa: F401  (load torch's HIP runtime before the library)
@@ -134,6 +135,7 @@ def last_error():
     return load().smx_last_error().decode("utf-8", "replace")
 
 
+@functools.lru_cache(maxsize=64, typed=True)  # a fixed rule of the library
 def tile_requirements(algo, epilogue, b_layout=SMX_B_KCONTIG):
     lib = load()
     tm, tn, tk = ctypes.c_int32(), ctypes.c_int32(), ctypes.c_int32()

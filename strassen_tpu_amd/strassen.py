@@ -58,6 +58,7 @@ from __future__ import annotations
 
 import contextlib
 import ctypes
+import functools
 import os
 import warnings
 
@@ -91,6 +92,8 @@ _EPILOGUES = ("swiglu", "geglu", "residual_add", "bias_add", "qk_norm_rope", "no
 
 def check_tiling(bm, bn, bk):
     """The reference's alignment rule (``strassen_pallas.py:127-140``)."""
+    if not (bm % (2 * SUBLANE) or bn % (2 * LANE) or bk % (2 * LANE)):
+        return
     requirements = (
         ("bm", bm, 2 * SUBLANE),
         ("bn", bn, 2 * LANE),
@@ -167,6 +170,38 @@ def strassen_kernel(kind):
         yield
     finally:
         STRASSEN_KERNEL = previous
+
+
+@functools.lru_cache(maxsize=512, typed=True)
+def _matmul_plan(device, algo, m, k, n, bm, bn, bk, epilogue, formula, block_permutation, out_f32, strassen_kernel,
+                 a_layout, a_dtype, passes, lda, ldr, aux, rope_head_dim, rope_eps, ldp):
+    """The descriptor of a packed call (as bytes) and the workspace it asks
+    for: all that the library derives from these values alone, so that a
+    repeated call neither fills the descriptor nor asks again. ``device`` is
+    part of the key because the launch shape follows its CU count."""
+    desc = _lib.SmxGemmDesc()
+    desc.m, desc.n, desc.k = m, n, k * passes
+    desc.lda, desc.ldb = lda, k * passes
+    desc.ldc = n // 2 if epilogue in ("swiglu", "geglu") else n
+    desc.ldr = ldr
+    desc.bm, desc.bn, desc.bk = bm, bn, bk
+    desc.algo = algo
+    desc.epilogue = _lib.SMX_EPI[epilogue]
+    desc.a_layout, desc.b_layout = a_layout, _lib.SMX_B_PACKED
+    desc.flags = _lib.SMX_FLAG_OUT_F32 if out_f32 else 0
+    if algo == 7 and strassen_kernel == "product_major":
+        desc.flags |= _lib.SMX_FLAG_PRODUCT_MAJOR
+    if algo == 7 and strassen_kernel == "product_major_rounds":
+        desc.flags |= _lib.SMX_FLAG_PRODUCT_MAJOR_ROUNDS
+    desc.formula = _lib.SMX_FORMULA[formula]
+    desc.block_permutation = block_permutation
+    desc.rope_head_dim, desc.rope_eps = rope_head_dim, rope_eps
+    desc.aux_f32 = aux
+    if ldp:  # an FP32 partial product: a stand-in address while sizes are asked for
+        desc.partial, desc.ldp = 16, ldp
+    need = ctypes.c_int64()
+    _lib.check(_lib.load().smx_matmul_workspace_bytes(desc, a_dtype, passes, ctypes.byref(need)))
+    return bytes(desc), need.value
 
 
 def _fits(algo, epilogue, bm, bn, bk, b_layout):
@@ -304,7 +339,8 @@ def _validate(a, b, *, bm, bn, bk, block_permutation, formula_variant,
         raise ValueError("block_permutation must be an integer from 0 through 7")
     if formula_variant not in ("classical", "dual", "powers"):
         raise ValueError("formula_variant must be 'classical', 'dual', or 'powers'")
-    classical_panels = tuple(sorted({int(p) for p in classical_panels}))
+    if classical_panels != ():
+        classical_panels = tuple(sorted({int(p) for p in classical_panels}))
     if epilogue is not None:
         _check_epilogue_name(epilogue)
         if formula_variant == "powers":
@@ -526,7 +562,7 @@ def _run(algo, a, b, *, bm, bn, bk, epilogue=None, residual=None, bias=None,
             if a.dtype == torch.float32:
                 a_dtype = _lib.SMX_DTYPE_F32
             a_ptr, lda = a, a.stride(0)
-        b_ptr, ldb = b.data, k * passes
+        b_ptr = b.data
     else:
         if a.stride(1) != 1 or a.stride(0) % 8 or a.data_ptr() % 16:
             a = a.contiguous()
@@ -534,28 +570,7 @@ def _run(algo, a, b, *, bm, bn, bk, epilogue=None, residual=None, bias=None,
             b = b.t().contiguous().t()
         bt = b.t()  # [N, K], rows contiguous
         a_ptr, b_ptr, lda, ldb = a, bt, a.stride(0), bt.stride(0)
-    out_cols = n // 2 if epilogue in ("swiglu", "geglu") else n
-    c = torch.empty((m, out_cols), dtype=out_dtype, device=a.device)
-    desc = _lib.SmxGemmDesc()
-    desc.m, desc.n, desc.k = m, n, k * passes
-    desc.lda, desc.ldb, desc.ldc = lda, ldb, c.stride(0)
-    desc.bm, desc.bn, desc.bk = bm, bn, bk
-    desc.algo = algo
-    desc.epilogue = _lib.SMX_EPI[epilogue]
-    desc.a_layout = a_layout
-    desc.b_layout = b_layout
-    desc.flags = _lib.SMX_FLAG_OUT_F32 if out_dtype == torch.float32 else 0
-    if algo == 7 and packed and STRASSEN_KERNEL == "product_major":
-        desc.flags |= _lib.SMX_FLAG_PRODUCT_MAJOR
-    if algo == 7 and packed and STRASSEN_KERNEL == "product_major_rounds":
-        desc.flags |= _lib.SMX_FLAG_PRODUCT_MAJOR_ROUNDS
-    desc.formula = _lib.SMX_FORMULA[formula]
-    desc.block_permutation = block_permutation
-    if partial is not None:
-        desc.partial, desc.ldp = partial.data_ptr(), partial.stride(0)
-    desc.rope_head_dim = rope_head_dim
-    desc.rope_eps = rope_eps
-    aux = 0
+    ldr = aux = 0
     if residual is not None:
         residual = _aux_tensor(residual)
         # the kernels read residual rows in 16-byte chunks
@@ -563,7 +578,7 @@ def _run(algo, a, b, *, bm, bn, bk, epilogue=None, residual=None, bias=None,
             residual = residual.contiguous()
         if residual.dtype == torch.float32:
             aux |= _lib.SMX_AUX_RESIDUAL_F32
-        desc.ldr = residual.stride(0)
+        ldr = residual.stride(0)
     if bias is not None:
         bias = _aux_tensor(bias.contiguous())
         if bias.dtype == torch.float32:
@@ -580,24 +595,39 @@ def _run(algo, a, b, *, bm, bn, bk, epilogue=None, residual=None, bias=None,
         rope_scale = rope_scale if rope_scale.data_ptr() % 16 == 0 else rope_scale.clone()
         if rope_scale.dtype == torch.float32:
             aux |= _lib.SMX_AUX_SCALE_F32
-    desc.aux_f32 = aux
-    # The library packs a row-major activation into the workspace, and asks
-    # for more of it when K is divided (FP32 shares of the output, summed by a
-    # second pass) or the product-major kernel takes the call (its two parked
-    # FP32 sets per tile).
-    stream = torch.cuda.current_stream(a.device).cuda_stream
-    pointers = (_lib.ptr(a_ptr), _lib.ptr(b_ptr), _lib.ptr(c), _lib.ptr(residual), _lib.ptr(bias), _lib.ptr(rope_cos),
-                _lib.ptr(rope_sin), _lib.ptr(rope_scale), stream)
-    need = ctypes.c_int64()
-    if not packed:
-        _lib.check(lib.smx_gemm(desc, *pointers))
-        return c
-    _lib.check(lib.smx_matmul_workspace_bytes(desc, a_dtype, passes, ctypes.byref(need)))
-    if need.value:
-        workspace = torch.empty(need.value, dtype=torch.uint8, device=a.device)
-        desc.workspace, desc.workspace_bytes = workspace.data_ptr(), need.value
-    rc = lib.smx_matmul(desc, a_dtype, passes, *pointers)
-    _lib.check(rc)
+    device = a.device
+    c = torch.empty((m, n // 2 if epilogue in ("swiglu", "geglu") else n), dtype=out_dtype, device=device)
+    stream = torch.cuda.current_stream(device).cuda_stream
+    pointers = [None if x is None else x.data_ptr()
+                for x in (a_ptr, b_ptr, c, residual, bias, rope_cos, rope_sin, rope_scale)]
+    if packed:
+        # The library packs a row-major activation into the workspace, and
+        # asks for more of it when K is divided (FP32 shares of the output,
+        # summed by a second pass) or the product-major kernel takes the call
+        # (its two parked FP32 sets per tile).
+        template, need = _matmul_plan(device.index, algo, m, k, n, bm, bn, bk, epilogue, formula, block_permutation,
+                                      out_dtype == torch.float32, STRASSEN_KERNEL, a_layout, a_dtype, passes, lda,
+                                      ldr, aux, rope_head_dim, float(rope_eps), 0 if partial is None else partial.stride(0))
+        desc = _lib.SmxGemmDesc.from_buffer_copy(template)
+        if partial is not None:
+            desc.partial = partial.data_ptr()
+        if need:
+            workspace = torch.empty(need, dtype=torch.uint8, device=device)
+            desc.workspace, desc.workspace_bytes = workspace.data_ptr(), need
+        rc = lib.smx_matmul(desc, a_dtype, passes, *pointers, stream)
+    else:
+        desc = _lib.SmxGemmDesc()
+        desc.m, desc.n, desc.k = m, n, k
+        desc.lda, desc.ldb, desc.ldc, desc.ldr = lda, ldb, c.stride(0), ldr
+        desc.bm, desc.bn, desc.bk = bm, bn, bk
+        desc.algo, desc.epilogue = algo, _lib.SMX_EPI[epilogue]
+        desc.a_layout, desc.b_layout = _lib.SMX_A_ROWMAJOR, b_layout
+        desc.flags = _lib.SMX_FLAG_OUT_F32 if out_dtype == torch.float32 else 0
+        desc.rope_head_dim, desc.rope_eps = rope_head_dim, rope_eps
+        desc.aux_f32 = aux
+        rc = lib.smx_gemm(desc, *pointers, stream)
+    if rc:
+        _lib.check(rc)
     return c
 
 

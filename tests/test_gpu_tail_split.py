@@ -417,3 +417,21 @@ def test_shares_that_do_not_divide_the_stages(algo, shape, tile):
     pa, pb = _pack(algo, a, b, tile)
     got, _ = abi_gemm(algo, pa, pb, m, n, k, tile, workspace=True, out_f32=True)
     assert np.array_equal(host(got), a @ b)
+
+
+@pytest.mark.parametrize("algo", [7, 8])
+@pytest.mark.parametrize("shape", [(256, 2048, 1280), (768, 2048, 2048), (256, 4096, 2560), (2048, 4096, 5120),
+                                   (2304, 2048, 8192)])
+def test_every_share_of_every_tile_runs_once(algo, shape):
+    """Shares are handed to the XCDs in eighths of (share, tile): launches of
+    5, 24, 10, 160 and 288 (32 split) tiles, with and without a multiple of 8
+    of tiles and of workgroups. Integer operands come out bit-exact, so every
+    share of every tile is formed and summed."""
+    m, k, n = shape
+    rng = np.random.default_rng(7 + algo + n)
+    a = rng.integers(-2, 3, (m, k)).astype(np.float32)
+    b = rng.integers(-2, 3, (k, n)).astype(np.float32)
+    pa, pb = _pack(algo, a, b, TILE)
+    got, need = abi_gemm(algo, pa, pb, m, n, k, TILE, workspace=True, out_f32=True)
+    assert need == _workspace_bytes(m, n, k)
+    assert np.array_equal(host(got), a @ b)

@@ -313,6 +313,9 @@ struct Params {
   // (kernel_stream.hpp): the FP32 [m, n] shares of a K-divided launch.
   void* park;
   int32_t epilogue;  // SMX_EPI_* of a kernel that chooses it at run time
+  // Workgroups behind those of the tiles (a launch of all tiles over full K)
+  // that read ahead (warm_panels).
+  int32_t warmers;
 };
 
 constexpr int kXcds = 8;

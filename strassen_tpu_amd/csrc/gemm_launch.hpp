@@ -24,10 +24,12 @@ int launch_strassen_epilogue(const Params& p, hipStream_t stream) {
       kern = split::gemm_split<SMX_EPI_NONE, kQuadPowers, kThin>;
     else
       return fail(SMX_ERR_INVALID, "fused epilogues require a quadrant-basis formula");
+  } else if (p.warmers) {
+    kern = split::gemm_split<kEpi, kQuadClassical, kThin, true>;
   } else {
     kern = split::gemm_split<kEpi, kQuadClassical, kThin>;
   }
-  return launch_kernel(kern, p, p.grid > 0 ? p.grid : p.tiles_m * p.tiles_n, lds, stream);
+  return launch_kernel(kern, p, (p.grid > 0 ? p.grid : p.tiles_m * p.tiles_n) + p.warmers, lds, stream);
 }
 
 template <bool kThin, int kEpi>

@@ -378,14 +378,50 @@ __device__ __forceinline__ void run_wave(const Params& p, const TileOrigin& o, i
   }
 }
 
-// kThin: a tiling whose bm/2 is not a multiple of 128 (ThinRows).
-template <int kEpi, int kQuad, bool kThin = false>
+// The body of the p.warmers workgroups that a launch of fewer tiles than CUs
+// puts on some of the CUs left over: they read the packed panels once, K position
+// by K position, so that the tiles' DMAs find them in the memory-side cache. A
+// tile's ring reaches two stages ahead, less than the slowest of a stage's
+// loads takes from HBM: with cold operands the tiles wait for memory whose
+// rate is far from used. Cold operands, 256 CUs: 160 tiles of K = 5120 181 us ->
+// 126, of K = 8192 273 -> 186, of K = 25600 721 -> 593. (The cubic, whose stages
+// take longer, gained 1-6% and goes without.) A warmer has four panels' stages
+// in flight.
+__device__ __forceinline__ void warm_panels(const Params& p, int nstages) {
+  constexpr int kStage = packed::Lay<7>::kStage, kLoads = kStage / (kThreads * 16), kAhead = 4;
+  static_assert(kStage % (kThreads * 16) == 0, "whole 16-byte loads");
+  const uint32_t panels = p.tiles_m + p.tiles_n, total = panels * nstages, step = p.warmers;
+  for (uint32_t u = blockIdx.x - p.tiles_m * p.tiles_n; u < total; u += kAhead * step) {
+    u32x4 v[kAhead][kLoads];
+#pragma unroll
+    for (int h = 0; h < kAhead; ++h) {
+      const uint32_t at = min(u + h * step, total - 1), stage = at / panels, panel = at - stage * panels;
+      const bool is_a = panel < (uint32_t)p.tiles_m;
+      const uint8_t* const from = reinterpret_cast<const uint8_t*>(is_a ? p.a : p.b) +
+                                  ((int64_t)(is_a ? panel : panel - p.tiles_m) * nstages + stage) * kStage +
+                                  threadIdx.x * 16;
+#pragma unroll
+      for (int i = 0; i < kLoads; ++i) v[h][i] = *reinterpret_cast<const u32x4*>(from + i * kThreads * 16);
+    }
+#pragma unroll
+    for (int h = 0; h < kAhead; ++h)
+#pragma unroll
+      for (int i = 0; i < kLoads; ++i) asm volatile("" ::"v"(v[h][i]));
+  }
+}
+
+// kThin: a tiling whose bm/2 is not a multiple of 128 (ThinRows). kWarm: a launch
+// with p.warmers; as a branch of the one kernel it cost short launches without
+// them 1.3%.
+template <int kEpi, int kQuad, bool kThin = false, bool kWarm = false>
 __global__ __launch_bounds__(kThreads, 1) void gemm_split(Params p) {
   using L = packed::Lay<7>;
   extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int nstages_all = (int)(p.k / (2 * TK));
+  if constexpr (kWarm)
+    if ((int)blockIdx.x >= p.tiles_m * p.tiles_n) return warm_panels(p, nstages_all);
   const WorkShare ws = work_share<1>(p, nstages_all);
   int tile_m, tile_n;
   tile_of(ws.tile, p.tiles_m, p.tiles_n, p.group_m, p.raster, tile_m, tile_n);

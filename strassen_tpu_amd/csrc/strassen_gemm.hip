@@ -495,7 +495,7 @@ constexpr int kSplitMinStages = 16;
 constexpr int kMaxKSplit = 16;
 constexpr int64_t kSplitMaxBytes = (int64_t)1 << 30;
 
-// Which tiles of a packed launch run as K shares. A launch runs one tile per
+// Which tiles of an smx_gemm launch run as K shares. A launch runs one tile per
 // CU and round: T tiles on C CUs make T / C whole rounds and a last round of
 // r = T mod C (r = T for a launch under one round). Those r tiles can run as
 // s shares of their K stages, s r workgroups in ceil(s r / C) rounds. In
@@ -545,7 +545,63 @@ int split_plan(const Params& p, SplitPlan* plan) {
   return SMX_OK;
 }
 
-int64_t split_bytes(const Params&, const SplitPlan& plan) {
+// Workgroups that read ahead (warm_panels) for a launch of whole tiles that
+// leaves an eighth of the CUs idle: that eighth. Fewer fall behind the tiles
+// and only add traffic (8 of 256: 224 tiles of K = 5120 186 us -> 271), more run
+// far ahead and take bandwidth from them (160 tiles of K = 5120, cold: none 175,
+// 16 166, 32 121, 64 129, 96 133; K = 25600: 721, 32 593, 48 644; operands still
+// in the memory-side cache: 118 without, 125 with 32). Strassen, classical formula.
+int warmers_of(const Params& p, int algo, int cus) {
+  if (algo != SMX_ALGO_STRASSEN || p.formula != SMX_FORMULA_CLASSICAL) return 0;
+  const int n = cus / 8;
+  return cus - p.tiles_m * p.tiles_n >= n ? n : 0;
+}
+
+// As split_plan, for smx_matmul's Strassen calls, from the times (us) that cold
+// operands give on MI355X. Over k of K a round of workgroups takes 0.031 k +
+// 12, however few they are: they wait for HBM. Shares add 25: their FP32 stores
+// and a second cold start; their second pass 3 and their bytes at 5 TB/s. A
+// launch with warmers takes 0.0182 k + 17 up to three eighths of the CUs and up
+// to 0.0252 at seven: fewer CUs leave each other memory and, within the chip's
+// power, clock. The cheapest by a twentieth is taken. split_plan's rule takes a
+// CU's rate as fixed. 256 CUs, measured (estimate): 80 tiles of K = 5120 in 3
+// shares 100 (106), 160 in 3 174 (183) and whole 126 (128), 384 with the last
+// 128 in 2 299 (303) and whole 328 (342); 160 of K = 8192 in 3 236 (246), whole
+// 186 (194); 80 of K = 25600 in 3 303 (317), whole 520 (499).
+// Below kMatmulSplitMinK the shares are split_plan's: the calls are short and the
+// plans within some us of each other (K = 2048, cold: 128 tiles 76 in two
+// shares, 80 whole; 384 156 and 153).
+constexpr int64_t kMatmulSplitMinK = 4096;
+
+int matmul_split_plan(const Params& p, int algo, SplitPlan* plan) {
+  if (algo != SMX_ALGO_STRASSEN || p.k < kMatmulSplitMinK) return split_plan(p, plan);
+  int cus = 0;
+  if (int rc = device_cus(&cus)) return rc;
+  const int tiles = p.tiles_m * p.tiles_n, r = tiles % cus;
+  *plan = SplitPlan{tiles, 0, 1};
+  if (p.partial || !split_setting() || r == 0) return SMX_OK;
+  const double k = (double)p.k;
+  auto rounds_us = [&](int64_t wgs, double depth) {
+    return (double)((wgs + cus - 1) / cus) * (depth * 0.031 + 12.0);
+  };
+  double whole = rounds_us(tiles, k);
+  if (warmers_of(p, algo, cus)) whole = k * (0.0182 + 0.014 * std::max(0.0, (double)tiles / cus - 0.375)) + 17.0;
+  const int stages = (int)(p.k / (2 * packed::TK));
+  const int64_t share_bytes = (int64_t)r * kSplitTileFloats * (int64_t)sizeof(float);
+  const int s_max = (int)std::min<int64_t>(std::min(kMaxKSplit, stages / kSplitMinStages), kSplitMaxBytes / share_bytes);
+  double best = 0.95 * whole;
+  for (int s = 2; s <= s_max; ++s) {
+    const double c = rounds_us(tiles - r, k) + rounds_us((int64_t)s * r, k / s) + 28.0 +
+                     (double)(s * share_bytes) / 5e6;
+    if (c < best) {
+      best = c;
+      *plan = SplitPlan{tiles - r, r, s};
+    }
+  }
+  return SMX_OK;
+}
+
+int64_t split_bytes(const SplitPlan& plan) {
   return (int64_t)plan.ksplit * plan.split * kSplitTileFloats * (int64_t)sizeof(float);
 }
 
@@ -604,9 +660,9 @@ int64_t pm_park_bytes(const Params& p) { return (int64_t)p.tiles_m * p.tiles_n *
 // Depth below which a SMX_FLAG_PRODUCT_MAJOR_ROUNDS call runs on the split
 // kernel alone. The product-major kernel's per-tile costs (two mid-kernel
 // epilogues, two parked sets) are fixed while its lead per unit of K is
-// small: on whole rounds (8192 x K x 16384, one MI355X) it takes 15% longer
-// than the split kernel at K = 1024, 3% at 2048, the same at 3072, 1% less
-// at 4096, 1-2% at 5120 and 10% at 25600.
+// small: on whole rounds (8192 x K x 16384, one MI355X) it takes 18% longer
+// than the split kernel at K = 1024, 4% at 2048, 1% less at 3072, 5% at 4096
+// and 13% at 8192.
 constexpr int64_t kPmRoundsMinK = 4096;
 
 // Product-major tile columns that a SMX_FLAG_PRODUCT_MAJOR_ROUNDS call runs on
@@ -652,9 +708,13 @@ struct Parts {
   bool rest = true;   // whether a split-kernel part follows
   Params head{};      // on pm_grid
   Params rest_p{};    // on packed_grid
+  SplitPlan split{};  // of the rest's K, with a workspace
 };
 
-int plan_parts(const Params& p, const smx_gemm_desc& d, Parts* out) {
+// The rule for the rest's K split: smx_gemm's (split_plan) or smx_matmul's.
+enum class SplitRule { kGemm, kMatmul };
+
+int plan_parts(const Params& p, const smx_gemm_desc& d, SplitRule rule, Parts* out) {
   Parts t;
   t.rest_p = p;
   if (pm_eligible(p, d)) {
@@ -678,23 +738,20 @@ int plan_parts(const Params& p, const smx_gemm_desc& d, Parts* out) {
       t.rest_p = column_part(p, d.epilogue, pcols, p.n / 2 - pcols);
     }
   }
-  if (t.rest) packed_grid(t.rest_p, d.algo);
+  if (t.rest) {
+    packed_grid(t.rest_p, d.algo);
+    if (int rc = rule == SplitRule::kGemm ? split_plan(t.rest_p, &t.split)
+                                          : matmul_split_plan(t.rest_p, d.algo, &t.split))
+      return rc;
+  }
   *out = t;
   return SMX_OK;
 }
 
 // Workspace bytes of a planned call: the head's parked sets and the rest's
-// K shares (split_plan), which run one after the other on one stream and
-// share the buffer.
-int parts_workspace(const Parts& t, int64_t* bytes) {
-  int64_t need = t.pm_cols ? pm_park_bytes(t.head) : 0;
-  if (t.rest) {
-    SplitPlan plan{};
-    if (int rc = split_plan(t.rest_p, &plan)) return rc;
-    if (plan.split) need = std::max(need, split_bytes(t.rest_p, plan));
-  }
-  *bytes = need;
-  return SMX_OK;
+// K shares, which run one after the other on one stream and share the buffer.
+int64_t parts_workspace(const Parts& t) {
+  return std::max(t.pm_cols ? pm_park_bytes(t.head) : 0, t.rest && t.split.split ? split_bytes(t.split) : 0);
 }
 
 // The workspace checks of a checked call, run before anything is launched
@@ -704,10 +761,9 @@ int parts_workspace(const Parts& t, int64_t* bytes) {
 int check_workspace(const Params& p, const smx_gemm_desc& d) {
   if (d.b_layout != SMX_B_PACKED) return SMX_OK;
   Parts t;
-  if (int rc = plan_parts(p, d, &t)) return rc;
+  if (int rc = plan_parts(p, d, SplitRule::kGemm, &t)) return rc;
   if (!t.pm_cols && !d.workspace) return SMX_OK;
-  int64_t need = 0;
-  if (int rc = parts_workspace(t, &need)) return rc;
+  const int64_t need = parts_workspace(t);
   if (t.pm_cols && (!d.workspace || d.workspace_bytes < need))
     return fail(SMX_ERR_INVALID,
                 "the product-major kernel needs workspace_bytes >= %lld (smx_gemm_workspace_bytes), got %lld",
@@ -718,41 +774,26 @@ int check_workspace(const Params& p, const smx_gemm_desc& d) {
   return SMX_OK;
 }
 
-int launch_rest(Params p, const smx_gemm_desc& d, hipStream_t s);
-
-// A packed call: a product-major head (plan_parts) parks two partial sets
-// per workgroup in the workspace; the rest runs as launch_rest says.
-int launch_gemm(Params p, const smx_gemm_desc& d, hipStream_t s) {
-  if (d.b_layout != SMX_B_PACKED)
-    return d.algo == SMX_ALGO_STRASSEN ? dispatch_v1<7>(p, d.epilogue, s) : dispatch_v1<8>(p, d.epilogue, s);
-  if (int rc = check_workspace(p, d)) return rc;
-  Parts t;
-  if (int rc = plan_parts(p, d, &t)) return rc;
-  if (t.pm_cols) {
-    Params q = t.head;
-    q.park = d.workspace;
-    if (int rc = launch_strassen_pm(q, d.epilogue, s)) return rc;
-  }
-  return t.rest ? launch_rest(t.rest_p, d, s) : SMX_OK;
-}
-
 // The split (or cubic) kernel's part of a packed call (on packed_grid), with
-// tiles split over K when a workspace is given (smx_gemm_desc.workspace,
-// split_plan): the whole tiles with the fused epilogue, then the split
-// tiles' K shares into the workspace (FP32, no epilogue), then split_fixup,
-// all on the caller's stream in that order.
-int launch_rest(Params p, const smx_gemm_desc& d, hipStream_t s) {
-  SplitPlan plan{p.tiles_m * p.tiles_n, 0, 1};
-  if (d.workspace)
-    if (int rc = split_plan(p, &plan)) return rc;
-  if (!plan.split) return launch_packed(p, d.algo, d.epilogue, s);
+// tiles split over K as `plan` says when a workspace is given: the whole
+// tiles with the fused epilogue, then the split tiles' K shares into the
+// workspace (FP32, no epilogue), then split_fixup, all on the caller's stream
+// in that order.
+int launch_rest(const Params& p, const smx_gemm_desc& d, const SplitPlan& plan, void* workspace, hipStream_t s) {
+  if (!workspace || !plan.split) {
+    int cus = 0;
+    if (int rc = device_cus(&cus)) return rc;
+    Params q = p;
+    q.warmers = warmers_of(p, d.algo, cus);
+    return launch_packed(q, d.algo, d.epilogue, s);
+  }
   if (plan.whole > 0) {
     Params q = p;
     q.grid = plan.whole;
     if (int rc = launch_packed(q, d.algo, d.epilogue, s)) return rc;
   }
   Params h = p;
-  h.c = d.workspace;
+  h.c = workspace;
   h.out_f32 = 1;
   h.residual = h.bias = nullptr;
   h.rope_cos = h.rope_sin = nullptr;
@@ -766,7 +807,27 @@ int launch_rest(Params p, const smx_gemm_desc& d, hipStream_t s) {
   f.ksplit = plan.ksplit;
   f.tile_base = plan.whole;
   f.split_stride = (int64_t)plan.split * kSplitTileFloats;
-  return launch_split_fixup(f, d.epilogue, (const float*)d.workspace, plan.split, s);
+  return launch_split_fixup(f, d.epilogue, (const float*)workspace, plan.split, s);
+}
+
+// A planned packed call: a product-major head parks two partial sets per
+// workgroup in the workspace; the rest runs as launch_rest says.
+int launch_parts(const Parts& t, const smx_gemm_desc& d, void* workspace, hipStream_t s) {
+  if (t.pm_cols) {
+    Params q = t.head;
+    q.park = workspace;
+    if (int rc = launch_strassen_pm(q, d.epilogue, s)) return rc;
+  }
+  return t.rest ? launch_rest(t.rest_p, d, t.split, workspace, s) : SMX_OK;
+}
+
+int launch_gemm(const Params& p, const smx_gemm_desc& d, hipStream_t s) {
+  if (d.b_layout != SMX_B_PACKED)
+    return d.algo == SMX_ALGO_STRASSEN ? dispatch_v1<7>(p, d.epilogue, s) : dispatch_v1<8>(p, d.epilogue, s);
+  if (int rc = check_workspace(p, d)) return rc;
+  Parts t;
+  if (int rc = plan_parts(p, d, SplitRule::kGemm, &t)) return rc;
+  return launch_parts(t, d, d.workspace, s);
 }
 
 // How smx_matmul runs a packed call on the streaming kernel (kernel_stream.hpp):
@@ -1070,8 +1131,9 @@ int smx_gemm_workspace_bytes(const smx_gemm_desc* d, int64_t* bytes) {
   if (int rc = gemm_params(d, x, x, const_cast<void*>(x), x, x, x, x, x, p)) return rc;
   if (d->b_layout != SMX_B_PACKED) return SMX_OK;
   Parts t;
-  if (int rc = plan_parts(p, *d, &t)) return rc;
-  return parts_workspace(t, bytes);
+  if (int rc = plan_parts(p, *d, SplitRule::kGemm, &t)) return rc;
+  *bytes = parts_workspace(t);
+  return SMX_OK;
 }
 
 int smx_gemm_noalloc(const smx_gemm_desc* d, const void* a, const void* b, void* c, const void* residual,
@@ -1121,6 +1183,7 @@ struct MatmulCall {
   smx_gemm_desc desc;
   Params p{};
   StreamPlan stream;
+  Parts parts;  // without a stream plan
   int64_t a_bytes = 0, gemm_bytes = 0;
 };
 
@@ -1151,9 +1214,9 @@ int matmul_call(const smx_gemm_desc* d, int32_t a_dtype, int32_t passes, const v
     t.gemm_bytes = stream_bytes(t.p, t.stream);
     return SMX_OK;
   }
-  Parts parts;
-  if (int rc = plan_parts(t.p, t.desc, &parts)) return rc;
-  return parts_workspace(parts, &t.gemm_bytes);
+  if (int rc = plan_parts(t.p, t.desc, SplitRule::kMatmul, &t.parts)) return rc;
+  t.gemm_bytes = parts_workspace(t.parts);
+  return SMX_OK;
 }
 
 }  // namespace
@@ -1193,11 +1256,9 @@ int smx_matmul(const smx_gemm_desc* d, int32_t a_dtype, int32_t passes, const vo
   } else if (!aligned16(a)) {
     return fail(SMX_ERR_INVALID, "A must be 16-byte aligned");
   }
-  call.p.a = (const uint16_t*)packed_a;
+  call.p.a = call.parts.head.a = call.parts.rest_p.a = (const uint16_t*)packed_a;
   if (call.stream.shape >= 0) return launch_stream_plan(call.p, call.desc, call.stream, workspace, (hipStream_t)stream);
-  call.desc.workspace = workspace;
-  call.desc.workspace_bytes = call.gemm_bytes;
-  return launch_gemm(call.p, call.desc, (hipStream_t)stream);
+  return launch_parts(call.parts, call.desc, workspace, (hipStream_t)stream);
 }
 
 int smx_norm_residual_add(int64_t m, int64_t n, const float* x, int64_t ldx, const void* residual, int64_t ldr,

@@ -435,3 +435,19 @@ def test_every_share_of_every_tile_runs_once(algo, shape):
     got, need = abi_gemm(algo, pa, pb, m, n, k, TILE, workspace=True, out_f32=True)
     assert need == _workspace_bytes(m, n, k)
     assert np.array_equal(host(got), a @ b)
+
+
+@pytest.mark.parametrize("algo", [7, 8])
+@pytest.mark.parametrize("m,k,n,bm", [(256, 512, 512, 256), (2048, 1024, 5120, 256), (2048, 512, 7168, 256),
+                                      (2304, 512, 6400, 256), (272, 1536, 2560, 16)])
+def test_launches_that_read_ahead_bit_exact(algo, m, k, n, bm):
+    """Launches that leave an eighth of the CUs to workgroups that read the
+    packed panels ahead (2, 160, 224 tiles, a thin tiling's padded rows), and one
+    that leaves too few (225): integer operands come out bit-exact."""
+    rng = np.random.default_rng(31 + algo + n)
+    a = rng.integers(-2, 3, (m, k)).astype(np.float32)
+    b = rng.integers(-2, 3, (k, n)).astype(np.float32)
+    tile = (bm, 256, 512)
+    pa, pb = _pack(algo, a, b, tile)
+    got, _ = abi_gemm(algo, pa, pb, m, n, k, tile, workspace=False, out_f32=True)
+    assert np.array_equal(host(got), a @ b)

@@ -37,13 +37,14 @@
 // one operand (the current product's) per stage.
 //
 // Waves: wave w owns all 128 product rows and columns 64 w .. + 63 of the
-// tile, 4 x 2 blocks of 32 x 32 per set; per 16 k it uses 4 A and 2 B
-// fragments for 8 MFMAs. A's fragments are shared by the four waves and go
+// tile, 8 x 4 blocks of 16 x 16 per set; per 32 k it uses 8 A and 4 B
+// fragments for 32 MFMAs of 16 x 16 x 32. A's fragments are shared by the four waves and go
 // through LDS; B's belong to one wave each and go straight into its
 // registers. LDS then carries 64 KB of reads and 16 KB of DMA writes per
 // 1024 cycles of MFMAs; with both operands in LDS and 64 x 128 waves it was
 // 96 and 48 KB, more than its 128 bytes a cycle. Gate|up call (8192 x 5120 x
-// 51200, SwiGLU): 3.488 -> 3.364 ms, the chip being power limited.
+// 51200, SwiGLU): 3.488 -> 3.364 ms; with the stage addresses kept
+// incrementally (Stream) and one wait per half step 3.30, power limited.
 //
 // Pipeline: a stage is kQ 16-k steps of one product. B is loaded one stage
 // ahead (kQ = 8: 2048 cycles of MFMAs), A's ring is refilled kSlots - 1

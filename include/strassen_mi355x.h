@@ -41,7 +41,7 @@
 extern "C" {
 #endif
 
-#define SMX_VERSION 13
+#define SMX_VERSION 14
 
 /* Status codes. */
 #define SMX_OK 0
@@ -334,6 +334,17 @@ int smx_norm_residual_add(int64_t m, int64_t n, const float* x, int64_t ldx, con
  */
 int smx_rms_norm(int64_t m, int64_t n, const void* x, int64_t ldx, const void* scale, int32_t dtypes, float eps,
                  void* out, int64_t ldo, void* stream);
+
+/*
+ * The same norm in two passes around row factors that the caller forms with
+ * the order of additions of its own choice: smx_row_squares writes x^2 in FP32 (x
+ * bf16 [m, n], out dense [m, n]), and smx_scale_rows out = x * factor_row * scale
+ * (factor [m] FP32: rsqrt(mean_row + eps)), rounded once to bf16. Widths,
+ * alignment and dtypes as for smx_rms_norm. Asynchronous on stream.
+ */
+int smx_row_squares(int64_t m, int64_t n, const void* x, int64_t ldx, float* out, void* stream);
+int smx_scale_rows(int64_t m, int64_t n, const void* x, int64_t ldx, const float* factor, const void* scale,
+                   int32_t dtypes, void* out, int64_t ldo, void* stream);
 
 /*
  * Second pass of the qk_norm_rope epilogue (strassen_pallas.py:793-835) for

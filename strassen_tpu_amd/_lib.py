@@ -60,7 +60,8 @@ SMX_QK_SCALE_F32 = 1
 SMX_QK_OUT_F32 = 4
 
 EXPORTS = ("smx_gemm", "smx_gemm_noalloc", "smx_gemm_workspace_bytes", "smx_matmul", "smx_matmul_workspace_bytes",
-           "smx_tile_requirements", "smx_packed_bytes", "smx_pack_operand", "smx_pack_rhs_transposed", "smx_norm_residual_add", "smx_rms_norm", "smx_qk_norm_rope", "smx_last_error", "smx_version")
+           "smx_tile_requirements", "smx_packed_bytes", "smx_pack_operand", "smx_pack_rhs_transposed", "smx_norm_residual_add", "smx_rms_norm",
+           "smx_row_squares", "smx_scale_rows", "smx_qk_norm_rope", "smx_last_error", "smx_version")
 
 
 class SmxGemmDesc(ctypes.Structure):
@@ -121,6 +122,10 @@ def load():
     lib.smx_norm_residual_add.restype = ctypes.c_int
     lib.smx_rms_norm.argtypes = [i64, i64, vp, i64, vp, i32, f32, vp, i64, vp]
     lib.smx_rms_norm.restype = ctypes.c_int
+    lib.smx_row_squares.argtypes = [i64, i64, vp, i64, vp, vp]
+    lib.smx_row_squares.restype = ctypes.c_int
+    lib.smx_scale_rows.argtypes = [i64, i64, vp, i64, vp, vp, i32, vp, i64, vp]
+    lib.smx_scale_rows.restype = ctypes.c_int
     lib.smx_qk_norm_rope.argtypes = [i64, i64, vp, i64, vp, vp, vp, i32, i32, i32, f32, vp, i64, vp]
     lib.smx_qk_norm_rope.restype = ctypes.c_int
     lib.smx_last_error.argtypes = []

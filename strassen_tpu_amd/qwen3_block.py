@@ -101,20 +101,27 @@ def rms_norm(x, scale, eps):
 
 
 def _row_rms_norm(x, scale, eps):
-    """``rms_norm`` of a block's hidden state ``[tokens, hidden]`` in one pass
-    on the device (``smx_rms_norm``), the fused arms' norm. Its callers feed it
-    to kernels that carry no gradient. Other layouts and types take the
-    torch form."""
+    """``rms_norm`` of a block's hidden state ``[tokens, hidden]``, the fused
+    arms' norm, with the same bits in three passes over memory instead of
+    torch's seven: the squares (``smx_row_squares``), torch's own mean over
+    them, whose order of additions is part of the result, and the scaling
+    (``smx_scale_rows``). Other layouts and types, and calls that record
+    gradients, take the torch form."""
     if (x.device.type != "cuda" or x.dtype != torch.bfloat16 or x.dim() != 2 or not x.is_contiguous()
             or scale.device != x.device or scale.dtype not in (torch.bfloat16, torch.float32)
             or not scale.is_contiguous() or tuple(scale.shape) != (x.shape[1],) or not x.numel() or x.shape[1] % 8
-            or x.data_ptr() % 16 or scale.data_ptr() % 16):
+            or x.data_ptr() % 16 or scale.data_ptr() % 16
+            or (torch.is_grad_enabled() and (x.requires_grad or scale.requires_grad))):
         return rms_norm(x, scale, eps)
-    out = torch.empty_like(x)
+    lib, (m, n) = _lib.load(), x.shape
     stream = torch.cuda.current_stream(x.device).cuda_stream
-    _lib.check(_lib.load().smx_rms_norm(x.shape[0], x.shape[1], _lib.ptr(x), x.stride(0), _lib.ptr(scale),
-                                        _lib.SMX_NRA_SCALE_F32 if scale.dtype == torch.float32 else 0, float(eps),
-                                        _lib.ptr(out), out.stride(0), stream))
+    squares = torch.empty((m, n), dtype=torch.float32, device=x.device)
+    _lib.check(lib.smx_row_squares(m, n, _lib.ptr(x), x.stride(0), _lib.ptr(squares), stream))
+    factor = torch.rsqrt(squares.mean(-1) + eps)
+    out = torch.empty_like(x)
+    _lib.check(lib.smx_scale_rows(m, n, _lib.ptr(x), x.stride(0), _lib.ptr(factor), _lib.ptr(scale),
+                                  _lib.SMX_NRA_SCALE_F32 if scale.dtype == torch.float32 else 0, _lib.ptr(out),
+                                  out.stride(0), stream))
     return out
 
 

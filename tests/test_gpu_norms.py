@@ -37,6 +37,40 @@ def test_rms_norm(m, n, scale_dtype):
     _ulp_close(qb.rms_norm(x, scale, 1e-6), want)
 
 
+@pytest.mark.parametrize("m,n", [(1, 8), (3, 2040), (64, 5120), (2, 8200), (8192, 5120), (1, 25600)])
+@pytest.mark.parametrize("scale_dtype", [torch.bfloat16, torch.float32])
+def test_block_norm_has_the_bits_of_the_torch_form(m, n, scale_dtype):
+    """Rows over 40 binades, zero rows, and rows with an infinity or a NaN."""
+    g = torch.Generator(device=DEV).manual_seed(m + n)
+    x = torch.randn(m, n, device=DEV, generator=g) * torch.exp2(torch.rand(m, 1, device=DEV, generator=g) * 40 - 20)
+    for row, value in ((1, 0.0), (2, float("inf")), (3, float("nan"))):
+        if row < m:
+            x[row, slice(None) if value == 0 else n // 2] = value
+    x = x.to(torch.bfloat16)
+    scale = torch.randn(n, device=DEV, generator=g).to(scale_dtype)
+    got, want = qb._row_rms_norm(x, scale, 1e-6), qb.rms_norm(x, scale, 1e-6)
+    assert torch.equal(got.isnan(), want.isnan())
+    assert torch.equal(got[~got.isnan()], want[~want.isnan()])
+
+
+def test_block_norm_records_gradients():
+    x = torch.randn(4, 128, device=DEV).to(torch.bfloat16).requires_grad_()
+    scale = torch.randn(128, device=DEV).to(torch.bfloat16)
+    qb._row_rms_norm(x, scale, 1e-6).float().sum().backward()
+    assert x.grad is not None
+
+
+def test_rms_norm_in_one_pass():
+    """smx_rms_norm itself, rows apart and at widths past the registers."""
+    for n in (2040, 8200):
+        x = torch.randn(3, n + 8, device=DEV).to(torch.bfloat16)[:, :n]
+        scale, out = torch.randn(n, device=DEV), torch.empty(3, n, dtype=torch.bfloat16, device=DEV)
+        _lib.check(_lib.load().smx_rms_norm(3, n, x.data_ptr(), x.stride(0), scale.data_ptr(), _lib.SMX_NRA_SCALE_F32,
+                                            1e-6, out.data_ptr(), n, torch.cuda.current_stream(DEV).cuda_stream))
+        x64 = x.double()
+        _ulp_close(out, x64 * torch.rsqrt(x64.square().mean(-1, keepdim=True) + 1e-6) * scale.double())
+
+
 def test_rms_norm_keeps_other_layouts():
     """Widths and views that are not whole 16-byte chunks take the torch form."""
     x = torch.randn(4, 100, device=DEV).to(torch.bfloat16)

@@ -236,9 +236,11 @@ int smx_gemm_workspace_bytes(const smx_gemm_desc* desc, int64_t* bytes);
  * the call packs into the workspace first. Launches with few product rows or
  * few tiles (decode-sized M, small squares) then run on the streaming
  * kernel, whose tiles are smaller and which takes operands straight from
- * memory to registers; other calls run as smx_gemm runs them (flags choose
- * the Strassen kernel; a Strassen call without
- * SMX_FLAG_PRODUCT_MAJOR_ROUNDS never takes the streaming kernel). Results
+ * memory to registers; other calls run as smx_gemm with its workspace runs them
+ * (flags choose the Strassen kernel; a Strassen call without
+ * SMX_FLAG_PRODUCT_MAJOR_ROUNDS never takes the streaming kernel), except
+ * that some launches that smx_gemm divides over K stay whole here, with idle
+ * CUs reading their operands ahead. smx_matmul_plan tells how a call runs. Results
  * match smx_gemm's up to the order of FP32 additions. desc->workspace must
  * hold smx_matmul_workspace_bytes(desc, ...) bytes (16-byte aligned; NULL
  * when that is 0); every argument is checked before anything is launched.
@@ -248,6 +250,23 @@ int smx_matmul(const smx_gemm_desc* desc, int32_t a_dtype, int32_t passes, const
                const void* residual, const void* bias, const void* rope_cos, const void* rope_sin,
                const void* rope_scale, void* stream);
 int smx_matmul_workspace_bytes(const smx_gemm_desc* desc, int32_t a_dtype, int32_t passes, int64_t* bytes);
+
+/*
+ * How smx_matmul runs a call on a device of cus compute units (0: the current
+ * device's; a count needs no device). Launches nothing; desc as for
+ * smx_matmul_workspace_bytes.
+ */
+typedef struct smx_matmul_launch {
+  int32_t streaming;    /* 1: the streaming kernel, 0: the tile kernels */
+  int32_t tile_rows;    /* product rows and columns of a workgroup's tile */
+  int32_t tile_cols;
+  int32_t head_columns; /* columns of 256 on the product-major kernel (those below: the rest) */
+  int32_t whole_tiles;  /* tiles over full K */
+  int32_t split_tiles;  /* tiles in `shares` shares of K each */
+  int32_t shares;
+  int32_t readers;      /* workgroups that read the packed operands ahead */
+} smx_matmul_launch;
+int smx_matmul_plan(const smx_gemm_desc* desc, int32_t a_dtype, int32_t passes, int32_t cus, smx_matmul_launch* plan);
 
 /* Tile granules of the kernels that serve (algo, epilogue, b_layout): bm
  * must be a multiple of 2*tm, bn of 2*tn, bk of 2*tk. Packed operands: 8, 128,

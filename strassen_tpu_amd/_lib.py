@@ -59,7 +59,7 @@ SMX_NRA_OUT_F32 = 4
 SMX_QK_SCALE_F32 = 1
 SMX_QK_OUT_F32 = 4
 
-EXPORTS = ("smx_gemm", "smx_gemm_noalloc", "smx_gemm_workspace_bytes", "smx_matmul", "smx_matmul_workspace_bytes",
+EXPORTS = ("smx_gemm", "smx_gemm_noalloc", "smx_gemm_workspace_bytes", "smx_matmul", "smx_matmul_workspace_bytes", "smx_matmul_plan",
            "smx_tile_requirements", "smx_packed_bytes", "smx_pack_operand", "smx_pack_rhs_transposed", "smx_norm_residual_add", "smx_rms_norm",
            "smx_row_squares", "smx_scale_rows", "smx_qk_norm_rope", "smx_last_error", "smx_version")
 
@@ -79,6 +79,13 @@ class SmxGemmDesc(ctypes.Structure):
         ("partial", ctypes.c_void_p), ("ldp", ctypes.c_int64),
         ("workspace", ctypes.c_void_p), ("workspace_bytes", ctypes.c_int64),
     ]
+
+
+class SmxMatmulLaunch(ctypes.Structure):
+    """``smx_matmul_launch``: how smx_matmul runs a call."""
+
+    _fields_ = [(name, ctypes.c_int32) for name in ("streaming", "tile_rows", "tile_cols", "head_columns",
+                                                    "whole_tiles", "split_tiles", "shares", "readers")]
 
 
 _lib = None
@@ -111,6 +118,8 @@ def load():
     lib.smx_matmul.restype = ctypes.c_int
     lib.smx_matmul_workspace_bytes.argtypes = [ctypes.POINTER(SmxGemmDesc), i32, i32, ctypes.POINTER(i64)]
     lib.smx_matmul_workspace_bytes.restype = ctypes.c_int
+    lib.smx_matmul_plan.argtypes = [ctypes.POINTER(SmxGemmDesc), i32, i32, i32, ctypes.POINTER(SmxMatmulLaunch)]
+    lib.smx_matmul_plan.restype = ctypes.c_int
     lib.smx_packed_bytes.argtypes = [i32, i64, i64, ctypes.POINTER(i64)]
     lib.smx_packed_bytes.restype = ctypes.c_int
     lib.smx_pack_operand.argtypes = [i32, i32, i32, i32, i64, i64, vp, i32, i32, i64, i32, i32, vp, i64, vp, vp]

@@ -470,6 +470,9 @@ int device_cus(int* cus) {
   return SMX_OK;
 }
 
+// The CUs a launch is planned for: those given, or the current device's.
+int planned_cus(int* cus) { return *cus > 0 ? SMX_OK : device_cus(cus); }
+
 // SMX_TAIL_SPLIT=0 keeps every tile of a launch over full K (for timing
 // the launch shapes against each other).
 bool split_setting() {
@@ -551,11 +554,10 @@ double split_cost(int s, int r, int cus, int64_t k) {
   return (double)rounds * (1.0 / (double)s + f) + (double)(s * r) * g;
 }
 
-int split_plan(const Params& p, SplitPlan* plan) {
+int split_plan(const Params& p, int cus, SplitPlan* plan) {
   *plan = SplitPlan{p.tiles_m * p.tiles_n, 0, 1};
   if (p.partial || !split_setting() || p.k < kSplitMinK) return SMX_OK;
-  int cus = 0;
-  if (int rc = device_cus(&cus)) return rc;
+  if (int rc = planned_cus(&cus)) return rc;
   const int tiles = p.tiles_m * p.tiles_n;
   const int r = tiles % cus;
   if (r == 0) return SMX_OK;
@@ -575,59 +577,43 @@ int split_plan(const Params& p, SplitPlan* plan) {
   return SMX_OK;
 }
 
-// Workgroups that read ahead (warm_panels) for a launch of whole tiles that
-// leaves an eighth of the CUs idle: that eighth. Fewer fall behind the tiles
-// and only add traffic (8 of 256: 224 tiles of K = 5120 186 us -> 271), more run
-// far ahead and take bandwidth from them (160 tiles of K = 5120, cold: none 175,
-// 16 166, 32 121, 64 129, 96 133; K = 25600: 721, 32 593, 48 644; operands still
-// in the memory-side cache: 118 without, 125 with 32). Strassen, classical formula.
+// Workgroups that read ahead (warm_panels) for a launch of whole Strassen tiles
+// in one round: an eighth of the CUs, where they are idle. Fewer fall behind
+// the tiles and only add traffic (8 of 256: 224 tiles of K = 5120 186 us -> 271),
+// more run far ahead and take bandwidth from them (160 tiles of K = 5120, cold:
+// none 175, 16 166, 32 121, 64 129, 96 133).
+//
+// They help as long as they keep ahead. A workgroup reads some 70 bytes a ns and
+// the tiles take a stage of every panel, 28 KB each, in the 0.58 us of its MFMAs:
+// 1.4 panels a workgroup, 44 on 256 CUs. Measured cold, without and with them (in
+// brackets with operands still in the memory-side cache), K = 5120: 8 x 20 tiles
+// 147 -> 120 us (114 -> 118), 4 x 34 142 -> 118 (106 -> 109), 5 x 32 144 -> 122,
+// 4 x 40, 44 panels, 142 -> 131; past the line 4 x 50 150 -> 151, 3 x 70 176 -> 198,
+// 1 x 160 184 -> 447, 1 x 196 210 -> 562. Over half the CUs the tile count must
+// also be a multiple of the XCDs: others are not gathered on them (xcd_order),
+// miss the L2 more and lose to the readers what they gain (3 x 44 149 -> 140 cold but
+// 120 -> 140 cached, 5 x 27 153 -> 142 but 125 -> 142).
 int warmers_of(const Params& p, int algo, int cus) {
   if (algo != SMX_ALGO_STRASSEN || p.formula != SMX_FORMULA_CLASSICAL) return 0;
-  const int n = cus / 8;
-  return cus - p.tiles_m * p.tiles_n >= n ? n : 0;
+  const int n = cus / 8, tiles = p.tiles_m * p.tiles_n, panels = p.tiles_m + p.tiles_n;
+  const bool gathered = 2 * tiles <= cus || tiles % kXcds == 0;
+  return cus - tiles >= n && 5 * panels <= 7 * n && gathered ? n : 0;
 }
 
-// As split_plan, for smx_matmul's Strassen calls, from the times (us) that cold
-// operands give on MI355X. Over k of K a round of workgroups takes 0.031 k +
-// 12, however few they are: they wait for HBM. Shares add 25: their FP32 stores
-// and a second cold start; their second pass 3 and their bytes at 5 TB/s. A
-// launch with warmers takes 0.0182 k + 17 up to three eighths of the CUs and up
-// to 0.0252 at seven: fewer CUs leave each other memory and, within the chip's
-// power, clock. The cheapest by a twentieth is taken. split_plan's rule takes a
-// CU's rate as fixed. 256 CUs, measured (estimate): 80 tiles of K = 5120 in 3
-// shares 100 (106), 160 in 3 174 (183) and whole 126 (128), 384 with the last
-// 128 in 2 299 (303) and whole 328 (342); 160 of K = 8192 in 3 236 (246), whole
-// 186 (194); 80 of K = 25600 in 3 303 (317), whole 520 (499).
-// Below kMatmulSplitMinK the shares are split_plan's: the calls are short and the
-// plans within some us of each other (K = 2048, cold: 128 tiles 76 in two
-// shares, 80 whole; 384 156 and 153).
-constexpr int64_t kMatmulSplitMinK = 4096;
+// As split_plan, for smx_matmul. A launch of more tiles than half the CUs has
+// shares for two rounds and more; up to kReadAheadMaxK whole tiles with the
+// others reading ahead are faster, where warmers_of allows them (split_plan's
+// shares, whole, cold us: 8 x 20 tiles K = 4096 136, 101; K = 8192 224, 183; 4 x 34
+// K = 12288 285, 267; at K = 25600, whose panels no cache holds, 8 x 17 tiles 579,
+// 642 and 4 x 40 581, 606). At up to half the CUs the shares fit one round and
+// stay (8 x 16 tiles K = 5120 121, 123; 5 x 16 82, 108).
+constexpr int64_t kReadAheadMaxK = 16384;
 
-int matmul_split_plan(const Params& p, int algo, SplitPlan* plan) {
-  if (algo != SMX_ALGO_STRASSEN || p.k < kMatmulSplitMinK) return split_plan(p, plan);
-  int cus = 0;
-  if (int rc = device_cus(&cus)) return rc;
-  const int tiles = p.tiles_m * p.tiles_n, r = tiles % cus;
-  *plan = SplitPlan{tiles, 0, 1};
-  if (p.partial || !split_setting() || r == 0) return SMX_OK;
-  const double k = (double)p.k;
-  auto rounds_us = [&](int64_t wgs, double depth) {
-    return (double)((wgs + cus - 1) / cus) * (depth * 0.031 + 12.0);
-  };
-  double whole = rounds_us(tiles, k);
-  if (warmers_of(p, algo, cus)) whole = k * (0.0182 + 0.014 * std::max(0.0, (double)tiles / cus - 0.375)) + 17.0;
-  const int stages = (int)(p.k / (2 * packed::TK));
-  const int64_t share_bytes = (int64_t)r * kSplitTileFloats * (int64_t)sizeof(float);
-  const int s_max = (int)std::min<int64_t>(std::min(kMaxKSplit, stages / kSplitMinStages), kSplitMaxBytes / share_bytes);
-  double best = 0.95 * whole;
-  for (int s = 2; s <= s_max; ++s) {
-    const double c = rounds_us(tiles - r, k) + rounds_us((int64_t)s * r, k / s) + 28.0 +
-                     (double)(s * share_bytes) / 5e6;
-    if (c < best) {
-      best = c;
-      *plan = SplitPlan{tiles - r, r, s};
-    }
-  }
+int matmul_split_plan(const Params& p, int algo, int cus, SplitPlan* plan) {
+  if (int rc = split_plan(p, cus, plan)) return rc;
+  if (!plan->split || plan->whole || p.k > kReadAheadMaxK) return SMX_OK;
+  if (int rc = planned_cus(&cus)) return rc;
+  if (2 * plan->split > cus && warmers_of(p, algo, cus)) *plan = SplitPlan{plan->split, 0, 1};
   return SMX_OK;
 }
 
@@ -744,7 +730,7 @@ struct Parts {
 // The rule for the rest's K split: smx_gemm's (split_plan) or smx_matmul's.
 enum class SplitRule { kGemm, kMatmul };
 
-int plan_parts(const Params& p, const smx_gemm_desc& d, SplitRule rule, Parts* out) {
+int plan_parts(const Params& p, const smx_gemm_desc& d, SplitRule rule, int cus, Parts* out) {
   Parts t;
   t.rest_p = p;
   if (pm_eligible(p, d)) {
@@ -752,8 +738,7 @@ int plan_parts(const Params& p, const smx_gemm_desc& d, SplitRule rule, Parts* o
     pm_grid(q);
     int cols = q.tiles_n;
     if (d.flags & SMX_FLAG_PRODUCT_MAJOR_ROUNDS) {
-      int cus = 0;
-      if (int rc = device_cus(&cus)) return rc;
+      if (int rc = planned_cus(&cus)) return rc;
       cols = pm_round_columns(q, cus);
     }
     if (cols == q.tiles_n) {
@@ -770,8 +755,8 @@ int plan_parts(const Params& p, const smx_gemm_desc& d, SplitRule rule, Parts* o
   }
   if (t.rest) {
     packed_grid(t.rest_p, d.algo);
-    if (int rc = rule == SplitRule::kGemm ? split_plan(t.rest_p, &t.split)
-                                          : matmul_split_plan(t.rest_p, d.algo, &t.split))
+    if (int rc = rule == SplitRule::kGemm ? split_plan(t.rest_p, cus, &t.split)
+                                          : matmul_split_plan(t.rest_p, d.algo, cus, &t.split))
       return rc;
   }
   *out = t;
@@ -791,7 +776,7 @@ int64_t parts_workspace(const Parts& t) {
 int check_workspace(const Params& p, const smx_gemm_desc& d) {
   if (d.b_layout != SMX_B_PACKED) return SMX_OK;
   Parts t;
-  if (int rc = plan_parts(p, d, SplitRule::kGemm, &t)) return rc;
+  if (int rc = plan_parts(p, d, SplitRule::kGemm, 0, &t)) return rc;
   if (!t.pm_cols && !d.workspace) return SMX_OK;
   const int64_t need = parts_workspace(t);
   if (t.pm_cols && (!d.workspace || d.workspace_bytes < need))
@@ -856,7 +841,7 @@ int launch_gemm(const Params& p, const smx_gemm_desc& d, hipStream_t s) {
     return d.algo == SMX_ALGO_STRASSEN ? dispatch_v1<7>(p, d.epilogue, s) : dispatch_v1<8>(p, d.epilogue, s);
   if (int rc = check_workspace(p, d)) return rc;
   Parts t;
-  if (int rc = plan_parts(p, d, SplitRule::kGemm, &t)) return rc;
+  if (int rc = plan_parts(p, d, SplitRule::kGemm, 0, &t)) return rc;
   return launch_parts(t, d, d.workspace, s);
 }
 
@@ -867,7 +852,7 @@ struct StreamPlan {
 };
 
 // Estimated time in us of a packed call on the 128 x 128 tile kernels (with
-// the K split that split_plan gives it): per tile and round 0.027 us of K
+// the K split that matmul_split_plan gives it): per tile and round 0.027 us of K
 // (Strassen) or 0.022 (cubic), three quarters of that while at most half the
 // CUs work, and 10 us around it; the packed weight at 4.4 TB/s; 8 us and the
 // shares' traffic for a split's second pass. Measured on MI355X, packed
@@ -903,11 +888,10 @@ double tile_kernel_us(const Params& p, int algo, int cus, const SplitPlan& plan,
 // kStreamMinStages stages.
 constexpr int kStreamMinStages = 8;
 
-int stream_plan(const Params& p, const smx_gemm_desc& d, StreamPlan* plan) {
+int stream_plan(const Params& p, const smx_gemm_desc& d, int cus, StreamPlan* plan) {
   *plan = StreamPlan{};
   if (p.partial || (d.algo == SMX_ALGO_STRASSEN && !(d.flags & SMX_FLAG_PRODUCT_MAJOR_ROUNDS))) return SMX_OK;
-  int cus = 0;
-  if (int rc = device_cus(&cus)) return rc;
+  if (int rc = planned_cus(&cus)) return rc;
   const int64_t prows = p.m / 2, stages = p.k / 32;
   const double nops = packed::nops_of(d.algo);
   const double packed_b = (double)p.n / 2 * (double)p.k / 2 * nops * 2;
@@ -916,7 +900,7 @@ int stream_plan(const Params& p, const smx_gemm_desc& d, StreamPlan* plan) {
   const int64_t whole_tiles = (int64_t)q.tiles_m * q.tiles_n;
   if (whole_tiles > cus) return SMX_OK;  // over one round of tiles
   SplitPlan split{};
-  if (int rc = split_plan(q, &split)) return rc;
+  if (int rc = matmul_split_plan(q, d.algo, cus, &split)) return rc;
   double best = 0.9 * tile_kernel_us(q, d.algo, cus, split, packed_b);
   for (int i = 0; i < kStreamShapes; ++i) {
     const StreamShape& t = kStreamShape[i];
@@ -1161,7 +1145,7 @@ int smx_gemm_workspace_bytes(const smx_gemm_desc* d, int64_t* bytes) {
   if (int rc = gemm_params(d, x, x, const_cast<void*>(x), x, x, x, x, x, p)) return rc;
   if (d->b_layout != SMX_B_PACKED) return SMX_OK;
   Parts t;
-  if (int rc = plan_parts(p, *d, SplitRule::kGemm, &t)) return rc;
+  if (int rc = plan_parts(p, *d, SplitRule::kGemm, 0, &t)) return rc;
   *bytes = parts_workspace(t);
   return SMX_OK;
 }
@@ -1218,7 +1202,7 @@ struct MatmulCall {
 };
 
 int matmul_call(const smx_gemm_desc* d, int32_t a_dtype, int32_t passes, const void* b, void* c, const void* residual,
-                const void* bias, const void* rope_cos, const void* rope_sin, const void* rope_scale,
+                const void* bias, const void* rope_cos, const void* rope_sin, const void* rope_scale, int cus,
                 MatmulCall* call) {
   if (!d) return fail(SMX_ERR_INVALID, "null descriptor");
   if (d->b_layout != SMX_B_PACKED) return fail(SMX_ERR_UNSUPPORTED, "smx_matmul takes a packed B (SMX_B_PACKED)");
@@ -1239,12 +1223,12 @@ int matmul_call(const smx_gemm_desc* d, int32_t a_dtype, int32_t passes, const v
     const int64_t bytes = packed::padded_product_rows(d->m) * (d->k / 2) * packed::nops_of(d->algo) * 2;
     t.a_bytes = (bytes + 255) / 256 * 256;
   }
-  if (int rc = stream_plan(t.p, t.desc, &t.stream)) return rc;
+  if (int rc = stream_plan(t.p, t.desc, cus, &t.stream)) return rc;
   if (t.stream.shape >= 0) {
     t.gemm_bytes = stream_bytes(t.p, t.stream);
     return SMX_OK;
   }
-  if (int rc = plan_parts(t.p, t.desc, SplitRule::kMatmul, &t.parts)) return rc;
+  if (int rc = plan_parts(t.p, t.desc, SplitRule::kMatmul, cus, &t.parts)) return rc;
   t.gemm_bytes = parts_workspace(t.parts);
   return SMX_OK;
 }
@@ -1259,8 +1243,38 @@ int smx_matmul_workspace_bytes(const smx_gemm_desc* d, int32_t a_dtype, int32_t 
   *bytes = 0;
   const void* x = kNoAllocScratchProbe;
   MatmulCall call;
-  if (int rc = matmul_call(d, a_dtype, passes, x, const_cast<void*>(x), x, x, x, x, x, &call)) return rc;
+  if (int rc = matmul_call(d, a_dtype, passes, x, const_cast<void*>(x), x, x, x, x, x, 0, &call)) return rc;
   *bytes = call.a_bytes + call.gemm_bytes;
+  return SMX_OK;
+}
+
+int smx_matmul_plan(const smx_gemm_desc* d, int32_t a_dtype, int32_t passes, int32_t cus, smx_matmul_launch* out) {
+  g_error[0] = 0;
+  if (!out) return fail(SMX_ERR_INVALID, "null output");
+  if (cus < 0) return fail(SMX_ERR_INVALID, "cus must be >= 0, got %d", cus);
+  *out = smx_matmul_launch{};
+  if (int rc = planned_cus(&cus)) return rc;
+  const void* x = kNoAllocScratchProbe;
+  MatmulCall call;
+  if (int rc = matmul_call(d, a_dtype, passes, x, const_cast<void*>(x), x, x, x, x, x, cus, &call)) return rc;
+  if (call.stream.shape >= 0) {
+    const StreamShape& t = kStreamShape[call.stream.shape];
+    out->streaming = 1;
+    out->tile_rows = 32 * t.rb;
+    out->tile_cols = 32 * t.cb;
+    out->shares = call.stream.shares;
+    const int64_t rows = (call.p.m / 2 + out->tile_rows - 1) / out->tile_rows, cols = call.p.n / 2 / out->tile_cols;
+    (out->shares > 1 ? out->split_tiles : out->whole_tiles) = (int32_t)(rows * cols);
+    return SMX_OK;
+  }
+  const Parts& t = call.parts;
+  out->tile_rows = packed::TM;
+  out->tile_cols = packed::TN;
+  out->head_columns = t.pm_cols;
+  out->shares = t.rest ? t.split.ksplit : 1;
+  out->whole_tiles = t.rest ? t.split.whole : 0;
+  out->split_tiles = t.rest ? t.split.split : 0;
+  out->readers = t.rest && !t.split.split ? warmers_of(t.rest_p, call.desc.algo, cus) : 0;
   return SMX_OK;
 }
 
@@ -1269,7 +1283,7 @@ int smx_matmul(const smx_gemm_desc* d, int32_t a_dtype, int32_t passes, const vo
                const void* rope_scale, void* stream) {
   g_error[0] = 0;
   MatmulCall call;
-  if (int rc = matmul_call(d, a_dtype, passes, b, c, residual, bias, rope_cos, rope_sin, rope_scale, &call)) return rc;
+  if (int rc = matmul_call(d, a_dtype, passes, b, c, residual, bias, rope_cos, rope_sin, rope_scale, 0, &call)) return rc;
   if (!a) return fail(SMX_ERR_INVALID, "null operand pointer");
   const int64_t need = call.a_bytes + call.gemm_bytes;
   if (need && (!d->workspace || !aligned16(d->workspace) || d->workspace_bytes < need))

@@ -451,3 +451,32 @@ def test_launches_that_read_ahead_bit_exact(algo, m, k, n, bm):
     pa, pb = _pack(algo, a, b, tile)
     got, _ = abi_gemm(algo, pa, pb, m, n, k, tile, workspace=False, out_f32=True)
     assert np.array_equal(host(got), a @ b)
+
+
+@pytest.mark.parametrize("m,k,n,bm", [(1024, 512, 8704, 256), (2048, 4096, 5120, 256), (2032, 2048, 5120, 16)])
+def test_matmul_reads_ahead_bit_exact(m, k, n, bm):
+    """strassen_matmul on launches that smx_matmul_plan runs whole with
+    read-ahead workgroups (136 tiles; 160; 160 of a thin tiling with padded rows),
+    the last two of which smx_gemm divides over K: integer operands come out
+    bit-exact, a fused residual included (one rounding of an exact sum)."""
+    tile = (bm, 256, 512)
+    d = _lib.SmxGemmDesc()
+    d.m, d.n, d.k, d.lda, d.ldb, d.ldc = m, n, k, k, k, n
+    d.bm, d.bn, d.bk = tile
+    d.algo, d.b_layout, d.flags = 7, _lib.SMX_B_PACKED, _lib.SMX_FLAG_PRODUCT_MAJOR_ROUNDS
+    plan = _lib.SmxMatmulLaunch()
+    _lib.check(_lib.load().smx_matmul_plan(d, _lib.SMX_DTYPE_BF16, 1, 0, ctypes.byref(plan)))
+    if torch.cuda.get_device_properties(DEV).multi_processor_count == 256:
+        assert plan.readers == 32 and plan.split_tiles == 0
+    rng = np.random.default_rng(n + m)
+    a = rng.integers(-2, 3, (m, k)).astype(np.float32)
+    b = rng.integers(-2, 3, (k, n)).astype(np.float32)
+    _, pb = _pack(7, a, b, tile)
+    want = torch.from_numpy(a).to(DEV).double() @ torch.from_numpy(b).to(DEV).double()
+    kw = dict(bm=tile[0], bn=tile[1], bk=tile[2])
+    for _ in range(2):  # cold, then cached operands
+        got = smx.strassen_matmul(dev(a), pb, output_dtype=torch.float32, **kw)
+        assert torch.equal(got.double(), want)
+    residual = torch.from_numpy(rng.integers(-64, 65, (m, n)).astype(np.float32)).to(DEV).to(torch.bfloat16)
+    got = smx.strassen_matmul(dev(a), pb, epilogue="residual_add", residual=residual, **kw)
+    assert torch.equal(got, (want + residual.double()).to(torch.bfloat16))

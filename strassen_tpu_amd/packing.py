@@ -112,7 +112,7 @@ def exact_schedule(nk, *, classical_panels=(), panel_schedule=None):
     when no panel is exact. The split into the two GEMMs is sized on the
     host, so a schedule held on the device is read back (one
     synchronisation)."""
-    if panel_schedule is None and classical_panels == ():
+    if panel_schedule is None and isinstance(classical_panels, tuple) and not classical_panels:
         return None
     if panel_schedule is not None:
         if isinstance(panel_schedule, ExactSchedule):

@@ -339,7 +339,7 @@ def _validate(a, b, *, bm, bn, bk, block_permutation, formula_variant,
         raise ValueError("block_permutation must be an integer from 0 through 7")
     if formula_variant not in ("classical", "dual", "powers"):
         raise ValueError("formula_variant must be 'classical', 'dual', or 'powers'")
-    if classical_panels != ():
+    if not (isinstance(classical_panels, tuple) and not classical_panels):  # any iterable of integers
         classical_panels = tuple(sorted({int(p) for p in classical_panels}))
     if epilogue is not None:
         _check_epilogue_name(epilogue)

@@ -3,6 +3,7 @@ checks (strassen_pallas.py:927-1047) raise the same exception types and
 messages, and unsupported research options fail loudly. No GPU is used: every
 case is rejected before a launch."""
 
+import numpy as np
 import pytest
 import torch
 
@@ -72,6 +73,20 @@ def test_exact_panel_argument_errors(kwargs, match):
     a, b = t(256, 512), t(512, 256)
     with pytest.raises(ValueError, match=match):
         smx.strassen_matmul(a, b, bm=256, bn=256, bk=512, **kwargs)
+
+
+@pytest.mark.parametrize("kind", [list, set, iter, np.array, torch.tensor, lambda x: np.array(x, dtype=np.int32)])
+@pytest.mark.parametrize("panels", [[], [1], [1, 0]])
+def test_classical_panels_of_any_iterable(kind, panels):
+    from strassen_tpu_amd.packing import exact_schedule
+
+    schedule = exact_schedule(4, classical_panels=kind(panels))
+    assert (schedule.exact if schedule else ()) == tuple(sorted(panels))
+    # the checks are passed, and the call is refused for its CPU tensors only
+    with pytest.raises(ValueError, match="HIP device"):
+        smx.strassen_matmul(t(256, 1024), t(1024, 256), bm=256, bn=256, bk=512, classical_panels=kind(panels))
+    with pytest.raises(ValueError, match="outside 0..1"):
+        smx.strassen_matmul(t(256, 1024), t(1024, 256), bm=256, bn=256, bk=512, classical_panels=kind(panels + [5]))
 
 
 def test_exact_schedule_resolution():

@@ -141,6 +141,17 @@ def rope_values(seq, head_dim, theta, device):
     return torch.cos(angles).to(torch.bfloat16), torch.sin(angles).to(torch.bfloat16)
 
 
+def _heads_readable_in_place(query, key, value):
+    """Whether the flash kernel takes these heads as they lie, each key and
+    value head shared among its query heads: bf16 heads of 128 in one batch and
+    sequence, key and value alike, every row a 16-byte-aligned run."""
+    b, s, heads, _ = query.shape
+    return (all(t.dtype == torch.bfloat16 and t.device == query.device and t.dim() == 4 and t.shape[:2] == (b, s)
+                and t.shape[3] == 128 and t.stride(3) == 1 and t.data_ptr() % 16 == 0
+                and all(t.stride(i) > 0 and t.stride(i) % 8 == 0 for i in range(3)) for t in (query, key, value))
+            and s > 0 and key.shape == value.shape and key.shape[2] > 0 and heads % key.shape[2] == 0)
+
+
 def attention(query, key, value):
     """Causal grouped-query attention, ``[batch, seq, heads, head_dim]`` in
     and out (``jax.nn.dot_product_attention(..., is_causal=True)``, ``:370-372``).
@@ -151,14 +162,12 @@ def attention(query, key, value):
 
     On the device the flash kernel reads the heads as they lie and shares
     each key and value head among its query heads; elsewhere, with gradients
-    to record or for shapes it may not take, they are laid out head by head
-    and repeated first.
+    to record or for operands it may not take so, they are laid out head by
+    head and repeated first.
     """
     from torch.nn.attention import SDPBackend, sdpa_kernel
 
-    if (query.device.type == "cuda" and query.dtype == torch.bfloat16 and query.shape[3] == 128
-            and query.shape[2] % key.shape[2] == 0 and query.shape[1] == key.shape[1] > 0
-            and all(t.stride(3) == 1 for t in (query, key, value))
+    if (query.device.type == "cuda" and _heads_readable_in_place(query, key, value)
             and not (torch.is_grad_enabled() and any(t.requires_grad for t in (query, key, value)))):
         with sdpa_kernel([SDPBackend.FLASH_ATTENTION, SDPBackend.EFFICIENT_ATTENTION]):
             out = torch.nn.functional.scaled_dot_product_attention(

@@ -51,6 +51,26 @@ def test_block_surface_checks():
     assert tuple(block.cos.shape) == (256, 128)
 
 
+def test_which_heads_are_read_in_place():
+    """Operands that the grouped flash call may not take as they lie are laid
+    out first: another value width or head count, misaligned or overlapping
+    rows, mixed types."""
+    def heads(h, width=128, pad=0, offset=0, dtype=torch.bfloat16):
+        wide = torch.zeros(2, 16, h, width + pad + offset, dtype=dtype)
+        return wide[..., offset:offset + width]
+
+    ok = qb._heads_readable_in_place
+    q, k = heads(8), heads(2)
+    assert ok(q, k, heads(2)) and ok(heads(8, pad=8), k, heads(2, offset=8))
+    assert ok(q.transpose(1, 2).contiguous().transpose(1, 2), k, k)  # head by head
+    assert not ok(q, k, heads(2, width=64)) and not ok(heads(8, 64), heads(2, 64), heads(2, 64))
+    assert not ok(q, k, heads(4)) and not ok(q, heads(3), heads(3))
+    assert not ok(heads(8, offset=1), k, k) and not ok(q, heads(2, pad=1), k) and not ok(q, k, heads(2, offset=4))
+    assert not ok(q, k[:, :8], k[:, :8]) and not ok(q, k[:1], k[:1])
+    assert not ok(q, heads(1).expand(2, 16, 2, 128), k)
+    assert not ok(q, k, heads(2, dtype=torch.float32)) and not ok(heads(8, dtype=torch.float16), k, k)
+
+
 def test_decoder_metrics_on_cpu_tensors():
     """The streamed decoder's metrics (device-agnostic torch) against numpy."""
     from strassen_tpu_amd import streamed_decoder as sd

@@ -111,3 +111,14 @@ def test_attention_reads_heads_in_place(heads, kv):
     with torch.enable_grad():
         want = qb.attention(q.detach().requires_grad_(), k, v).detach()  # laid out and repeated
     assert torch.equal(qb.attention(q, k, v), want)
+
+
+@pytest.mark.parametrize("offset,pad", [(0, 8), (8, 0), (1, 7), (0, 1)])
+def test_attention_on_views(offset, pad):
+    """Heads inside wider rows: read in place where their rows are aligned, laid
+    out first where they are not, with the same bits."""
+    g = torch.Generator(device=DEV).manual_seed(2)
+    q, k, v = (torch.randn(2, 128, h, 128 + offset + pad, device=DEV, generator=g).to(torch.bfloat16)
+               [..., offset:offset + 128] for h in (8, 2, 2))
+    want = qb.attention(*(t.contiguous() for t in (q, k, v)))
+    assert torch.equal(qb.attention(q, k, v), want)

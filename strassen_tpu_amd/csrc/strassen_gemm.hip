@@ -178,7 +178,10 @@ int launch_pack(const void* src, bool src_f32, bool transposed, int64_t ld, int6
   const packed::PackGeom g{(uint32_t)rows, (uint32_t)tile_rows, (uint32_t)tile_rows / 2, (uint32_t)bk,
                            (uint32_t)bk / 2, (uint32_t)nsrc};
   if (transposed) {
-    if (!src_f32 && ld % 8 == 0) {
+    // pack_cols moves whole 128-byte lines; A's rows between them (ld % 64) it
+    // reads twice, and the gather is faster (A stored 4096 x 5120: whole lines 18.4 us,
+    // gathered 20.1; ld 5128 23.3 and 19.7). A row-major B is worth it either way.
+    if (!src_f32 && ld % (kSide == 0 ? 64 : 8) == 0) {
       hipLaunchKernelGGL((packed::pack_cols<kAlgo, kSide>), dim3((unsigned)blocks_of(8)), dim3(256), 0, stream,
                          (const uint16_t*)src, ld, g, formula, perm, panels, src_panels, out);
       return check_launch();

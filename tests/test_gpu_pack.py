@@ -52,8 +52,8 @@ def test_row_major_right_operand_packs_as_the_transposed_one(algo, perm, dtype, 
 @pytest.mark.parametrize("m,bm", [(16, 16), (144, 48), (512, 256)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_transposed_left_operand_with_any_row_stride(dtype, m, bm, ld_pad):
-    """Row strides that are no multiple of 16 bytes take the gathering
-    kernel, the others the one that moves 16-byte chunks."""
+    """Row strides that are not whole 128-byte lines take the gathering kernel,
+    the others the one that moves 16-byte chunks."""
     k = 576
     a = _source(m, k, dtype)
     wide = torch.zeros(k, m + ld_pad, dtype=dtype, device=DEV)
@@ -61,6 +61,19 @@ def test_transposed_left_operand_with_any_row_stride(dtype, m, bm, ld_pad):
     kw = dict(algo=7, tile_rows=bm, bk=64)
     want = pack_operand(a, side="lhs", **kw)
     got = pack_operand(wide[:, :m], side="lhs_t", **kw)
+    assert torch.equal(got.data.view(torch.int16), want.data.view(torch.int16))
+
+
+@pytest.mark.parametrize("algo", [7, 8])
+@pytest.mark.parametrize("m,bm,ld", [(16, 16, 64), (144, 48, 192), (512, 256, 512), (512, 256, 576)])
+def test_transposed_left_operand_in_whole_lines(algo, m, bm, ld):
+    """Row strides of whole 128-byte lines, which the 16-byte-chunk kernel
+    takes, with padding rows in the last product tile."""
+    a = _source(m, 576, torch.bfloat16)
+    wide = torch.zeros(576, ld, dtype=torch.bfloat16, device=DEV)
+    wide[:, :m] = a.t()
+    kw = dict(algo=algo, tile_rows=bm, bk=64)
+    want, got = pack_operand(a, side="lhs", **kw), pack_operand(wide[:, :m], side="lhs_t", **kw)
     assert torch.equal(got.data.view(torch.int16), want.data.view(torch.int16))
 
 

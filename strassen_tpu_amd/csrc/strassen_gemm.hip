@@ -914,8 +914,8 @@ int stream_plan(const Params& p, const smx_gemm_desc& d, int cus, StreamPlan* pl
     if (rows > 1 && whole_tiles > cus / 4) continue;
     if (d.epilogue == SMX_EPI_QK_NORM_ROPE && t.cb < 2) continue;  // a head is 64 columns of a half
     const int64_t tiles = rows * (p.n / (64 * t.cb));
-    const int64_t shares = std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(cus / tiles, kMaxKSplit),
-                                                                  stages / kStreamMinStages));
+    const int64_t shares = !split_setting() ? 1 : std::max<int64_t>(
+        1, std::min<int64_t>(std::min<int64_t>(cus / tiles, kMaxKSplit), stages / kStreamMinStages));
     const int64_t rounds = (tiles * shares + cus - 1) / cus;
     const double kb_per_stage = t.algo == SMX_ALGO_STRASSEN ? 7.0 * (t.rb + t.cb) : 4.0 * (2 * t.rb + t.cb);
     const double wg_us = (double)rounds * ((stages + shares - 1) / shares) * kb_per_stage * 1.024 / (rows > 1 ? 70 : 57);

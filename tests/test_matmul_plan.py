@@ -4,6 +4,9 @@ GPU; what the plans compute is checked in test_gpu_stream.py and
 test_gpu_tail_split.py."""
 
 import ctypes
+import os
+import subprocess
+import sys
 
 import pytest
 
@@ -82,6 +85,23 @@ def test_plans_cover_the_call(algo, cus):
                 assert p.readers == 0 or rows * cols + p.readers <= cus
                 if algo == 8:
                     assert not p.readers and not p.head_columns
+
+
+def test_tail_split_off_keeps_every_tile_whole():
+    """SMX_TAIL_SPLIT=0 (read once per process): no kernel divides K."""
+    script = """
+import test_matmul_plan as t
+for algo in (7, 8):
+    for m in (16, 80, 256, 1024, 2048):
+        for n in (256, 5120, 17664):
+            for k in (512, 4608, 25600):
+                p = t.plan(m, k, n, algo=algo)
+                assert p.shares == 1 and p.split_tiles == 0, (algo, m, k, n)
+"""
+    here = os.path.dirname(os.path.abspath(__file__))
+    env = dict(os.environ, SMX_TAIL_SPLIT="0",
+               PYTHONPATH=os.pathsep.join([here, os.path.dirname(here), os.environ.get("PYTHONPATH", "")]))
+    subprocess.run([sys.executable, "-c", script], env=env, check=True)
 
 
 def test_plan_checks_its_arguments():

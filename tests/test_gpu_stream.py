@@ -1,9 +1,10 @@
 """GPU parity of the streaming kernel (kernel_stream.hpp), which smx_matmul runs
-on launches of few product rows or few tiles: every tiling it has, at its
-edges (padding rows, the last columns, K in one share and in several),
+on launches of few product rows or few tiles: every tiling it has, with K in
+one share and in several, and its edges (padding rows, the last columns),
 against exact integer products, and every epilogue, formula and block
 permutation against the 128 x 128 tile kernels (smx_gemm on the same
-operands) within one bf16 ulp.
+operands) within one bf16 ulp. That these calls run on it is checked in
+test_matmul_plan.py.
 """
 
 import ctypes
@@ -17,12 +18,13 @@ import strassen_tpu_amd as smx
 from strassen_tpu_amd import _lib
 from test_gpu_parity import DEV, _qk_problem, assert_ulp_close, dev, dev_weight, host, say
 from test_gpu_tail_split import _pack, _problem, abi_gemm
+from test_matmul_plan import plan as launch_plan
 
 pytestmark = pytest.mark.gpu
 
 # (m, k, n), tile: product rows M/2 of 8 and 32 (one 32-row block, the second
-# with more columns than 256 tiles of 64), 40 and 64 (two), 72 and 128 (four),
-# then several tile rows: 136 (padding rows in the last) and 512.
+# with more columns than 256 tiles of 64), 40, 64, 72, 128 and 136 (padding rows
+# in the last tile row) and 512.
 SHAPES = [
     ((16, 512, 256), (16, 256, 512)),
     ((64, 4608, 1024), (64, 512, 512)),
@@ -33,6 +35,25 @@ SHAPES = [
     ((256, 512, 768), (256, 256, 512)),
     ((272, 1024, 512), (272, 256, 512)),
     ((1024, 1024, 1024), (1024, 1024, 512)),
+]
+
+
+# algo, (m, k, n), the tiling that 256 CUs get: product rows and columns per
+# workgroup, shares of K. One tile row (M/2 up to the tile's rows) loads B past
+# the L2, several read it through. Row tiles of 16: M/2 of 8, 40 and 72 leaves
+# padding rows in the last 32-row block, and in the second of a tile of two.
+TILINGS = [
+    (7, (16, 512, 256), (32, 64, 2)), (7, (16, 512, 17664), (32, 64, 1)),
+    (7, (16, 3072, 17664), (32, 128, 3)), (7, (16, 512, 33792), (32, 128, 1)),
+    (7, (80, 2048, 2816), (64, 64, 8)), (7, (80, 512, 17664), (64, 64, 1)),
+    (7, (80, 1536, 17664), (64, 128, 3)), (7, (80, 512, 33792), (64, 128, 1)),
+    (7, (80, 512, 256), (32, 32, 2)), (7, (80, 512, 4352), (32, 32, 1)),
+    (7, (144, 2048, 1536), (64, 64, 8)), (7, (144, 512, 12288), (64, 64, 1)),
+    (8, (16, 512, 256), (32, 64, 2)), (8, (16, 512, 17664), (32, 64, 1)),
+    (8, (16, 1024, 12288), (32, 128, 4)), (8, (16, 512, 33792), (32, 128, 1)),
+    (8, (80, 2048, 2816), (64, 64, 8)), (8, (80, 512, 17664), (64, 64, 1)),
+    (8, (80, 512, 256), (32, 32, 2)), (8, (80, 512, 4352), (32, 32, 1)),
+    (8, (144, 1536, 2048), (64, 64, 6)), (8, (144, 512, 12288), (64, 64, 1)),
 ]
 
 
@@ -62,6 +83,21 @@ def test_integer_products_are_exact(algo, shape, tile):
     for left in (dev(a), pa):  # packed by the call, and packed before it
         got = _call(algo, left, pb, tile, output_dtype=torch.float32)
         assert torch.equal(got.double(), want)
+
+
+@pytest.mark.parametrize("algo,shape,tiling", TILINGS)
+def test_every_tiling_is_exact(algo, shape, tiling):
+    m, k, n = shape
+    plan = launch_plan(m, k, n, algo=algo, bm=16, cus=0)  # this device's
+    if torch.cuda.get_device_properties(DEV).multi_processor_count == 256:
+        assert plan.streaming and (plan.tile_rows, plan.tile_cols, plan.shares) == tiling
+    g = torch.Generator(device=DEV).manual_seed(m + n + k)
+    a = torch.randint(-2, 3, (m, k), device=DEV, generator=g).to(torch.bfloat16)
+    b = torch.randint(-2, 3, (n, k), device=DEV, generator=g).to(torch.bfloat16).t()
+    want = a.double() @ b.double()
+    layout = smx.strassen_weight_layout if algo == 7 else smx.cubic_weight_layout
+    got = _call(algo, a, layout(b, 256, 512), (16, 256, 512), output_dtype=torch.float32)
+    assert torch.equal(got.double(), want)
 
 
 @pytest.mark.parametrize("epilogue", ["swiglu", "geglu", "residual_add", "bias_add"])

@@ -87,6 +87,36 @@ def test_plans_cover_the_call(algo, cus):
                     assert not p.readers and not p.head_columns
 
 
+def test_streaming_tests_reach_every_tiling():
+    """The calls of test_gpu_stream.py run on the streaming kernel, and its
+    tilings are all those that a grid of calls gets, each with K in one share
+    and in several."""
+    import test_gpu_stream as g
+
+    for algo, (m, k, n), tiling in g.TILINGS:
+        p = plan(m, k, n, algo=algo, bm=16)
+        assert p.streaming and (p.tile_rows, p.tile_cols, p.shares) == tiling
+    key = lambda algo, m, rows, cols, shares: (algo, rows, cols, m // 2 <= rows, shares > 1)  # noqa: E731
+    tested = {key(algo, m, *tiling) for algo, (m, _, _), tiling in g.TILINGS}
+    for algo in (7, 8):
+        for m in (16, 64, 80, 128, 144, 256, 272, 1024):
+            for n in [256, 512, 1024, 1536, 2816, 4352, 5120, 8192, 12288, 17664, 25600, 33792, 51200]:
+                for k in (512, 1024, 2048, 4608, 10240, 25600):
+                    p = plan(m, k, n, algo=algo, bm=16)
+                    if p.streaming:
+                        assert key(algo, m, p.tile_rows, p.tile_cols, p.shares) in tested, (algo, m, k, n)
+    for algo in (7, 8):
+        for (m, k, n), (bm, bn, _) in g.SHAPES:
+            assert plan(m, k, n, algo=algo, bm=bm, bn=bn).streaming
+        for m, k, n, bm in ((48, 4608, 512, 16), (272, 512, 512, 272)):
+            for epilogue in ("swiglu", "geglu", "residual_add", "bias_add"):
+                assert plan(m, k, n, algo=algo, bm=bm, epilogue=epilogue).streaming
+        assert plan(48, 2048, 1024, algo=algo, bm=16, epilogue="qk_norm_rope").streaming
+    for m, k in ((16, 512), (272, 4608)):
+        for formula in _lib.SMX_FORMULA:
+            assert plan(m, k, 512, bm=m, formula=formula).streaming
+
+
 def test_tail_split_off_keeps_every_tile_whole():
     """SMX_TAIL_SPLIT=0 (read once per process): no kernel divides K."""
     script = """

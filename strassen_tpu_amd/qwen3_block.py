@@ -28,6 +28,7 @@ from __future__ import annotations
 import dataclasses
 
 import torch
+from torch.utils._python_dispatch import _get_current_dispatch_mode
 
 from . import _lib
 from .layouts import (rope_layout_tables, rope_layout_to_heads, rope_scale_layout, rope_weight_layout,
@@ -144,12 +145,21 @@ def rope_values(seq, head_dim, theta, device):
 def _heads_readable_in_place(query, key, value):
     """Whether the flash kernel takes these heads as they lie, each key and
     value head shared among its query heads: bf16 heads of 128 in one batch and
-    sequence, key and value alike, every row a 16-byte-aligned run."""
+    sequence, key and value alike, every row a 16-byte-aligned run. Never for
+    operands without an address of their own (batched by ``vmap``, fake, other
+    tensor types) and while a call is traced, where these are not the tensors that
+    it will run on."""
+    if (torch.compiler.is_compiling() or _get_current_dispatch_mode() is not None
+            or any(type(t) is not torch.Tensor for t in (query, key, value))):
+        return False
     b, s, heads, _ = query.shape
-    return (all(t.dtype == torch.bfloat16 and t.device == query.device and t.dim() == 4 and t.shape[:2] == (b, s)
-                and t.shape[3] == 128 and t.stride(3) == 1 and t.data_ptr() % 16 == 0
-                and all(t.stride(i) > 0 and t.stride(i) % 8 == 0 for i in range(3)) for t in (query, key, value))
-            and s > 0 and key.shape == value.shape and key.shape[2] > 0 and heads % key.shape[2] == 0)
+    try:
+        rows = all(t.dtype == torch.bfloat16 and t.device == query.device and t.dim() == 4 and t.shape[:2] == (b, s)
+                   and t.shape[3] == 128 and t.stride(3) == 1 and t.data_ptr() % 16 == 0
+                   and all(t.stride(i) > 0 and t.stride(i) % 8 == 0 for i in range(3)) for t in (query, key, value))
+    except RuntimeError:  # data_ptr of a batched tensor
+        return False
+    return rows and s > 0 and key.shape == value.shape and key.shape[2] > 0 and heads % key.shape[2] == 0
 
 
 def attention(query, key, value):

@@ -71,6 +71,30 @@ def test_which_heads_are_read_in_place():
     assert not ok(q, k, heads(2, dtype=torch.float32)) and not ok(heads(8, dtype=torch.float16), k, k)
 
 
+def test_heads_are_laid_out_under_transforms():
+    """Batched and fake tensors have no address to look at, and a traced call
+    runs on other tensors later: neither raises, both take the general form."""
+    from torch._subclasses import FakeTensorMode
+    from torch.fx.experimental.proxy_tensor import make_fx
+
+    q, k = torch.zeros(2, 16, 8, 128, dtype=torch.bfloat16), torch.zeros(2, 16, 2, 128, dtype=torch.bfloat16)
+    seen = []
+
+    def look(q, k):
+        seen.append(qb._heads_readable_in_place(q, k, k))
+        return q * 1
+
+    assert (look(q, k), seen.pop())[1]
+    torch.vmap(look)(q[None].repeat(3, 1, 1, 1, 1), k[None].repeat(3, 1, 1, 1, 1))
+    for mode in ("real", "fake", "symbolic"):
+        make_fx(look, tracing_mode=mode)(q, k)
+    with FakeTensorMode() as fake:
+        fakes = fake.from_tensor(q), fake.from_tensor(k)
+        look(*fakes)
+    look(*fakes)
+    assert seen == [False] * 6
+
+
 def test_decoder_metrics_on_cpu_tensors():
     """The streamed decoder's metrics (device-agnostic torch) against numpy."""
     from strassen_tpu_amd import streamed_decoder as sd

@@ -122,3 +122,17 @@ def test_attention_on_views(offset, pad):
                [..., offset:offset + 128] for h in (8, 2, 2))
     want = qb.attention(*(t.contiguous() for t in (q, k, v)))
     assert torch.equal(qb.attention(q, k, v), want)
+
+
+def test_attention_under_transforms():
+    """Batched by vmap and traced, with the bits of the plain call."""
+    from torch.fx.experimental.proxy_tensor import make_fx
+
+    g = torch.Generator(device=DEV).manual_seed(3)
+    q, k, v = (torch.randn(3, 2, 64, h, 128, device=DEV, generator=g).to(torch.bfloat16) for h in (8, 2, 2))
+    want = torch.stack([qb.attention(*t) for t in zip(q, k, v)])
+    assert torch.equal(torch.vmap(qb.attention)(q, k, v), want)
+    traced = make_fx(qb.attention, tracing_mode="fake")(q[0], k[0], v[0])
+    # the traced call lays out what it is given: rows that are not 16-byte aligned too
+    odd = [torch.nn.functional.pad(t[1], (1, 7))[..., 1:129] for t in (q, k, v)]
+    assert torch.equal(traced(*odd), want[1])

@@ -173,25 +173,17 @@ def ptr(t):
     return None if t is None else ctypes.c_void_p(t.data_ptr())
 
 
-def k_shares(m, k, n, tile, algo=SMX_ALGO_STRASSEN):
-    """K shares smx_gemm gives the split tiles of a packed (m, k, n) launch
-    on the current device (1: no split), from smx_gemm_workspace_bytes."""
-    lib = load()
+def k_shares(m, k, n, tile, algo=SMX_ALGO_STRASSEN, cus=0):
+    """K shares of the tiles that a packed (m, k, n) call divides (1: none), on
+    whichever kernel it runs (smx_matmul_plan), for ``cus`` compute units (0: the
+    current device's)."""
     d = SmxGemmDesc()
     d.m, d.n, d.k = m, n, k
     d.lda, d.ldb, d.ldc = k, k, n
     d.bm, d.bn, d.bk = tile
     d.algo = algo
+    d.flags = SMX_FLAG_PRODUCT_MAJOR_ROUNDS if algo == SMX_ALGO_STRASSEN else 0
     d.a_layout, d.b_layout = SMX_A_PACKED, SMX_B_PACKED
-    d.rope_head_dim, d.rope_eps = 128, 1e-6
-    need = ctypes.c_int64()
-    check(lib.smx_gemm_workspace_bytes(d, ctypes.byref(need)))
-    if not need.value:
-        return 1
-    # The workspace holds one 256 x 256 FP32 block per share and split tile;
-    # the split tiles are the last round's (128 x 128 product tiles, one per CU
-    # and round).
-    cus = torch.cuda.get_device_properties(torch.cuda.current_device()).multi_processor_count
-    tiles = -(-(m // 2) // 128) * ((n // 2) // 128)
-    split = tiles % cus or cus
-    return need.value // (split * 256 * 256 * 4)
+    launch = SmxMatmulLaunch()
+    check(load().smx_matmul_plan(d, SMX_DTYPE_BF16, 1, cus, ctypes.byref(launch)))
+    return launch.shares

@@ -381,9 +381,9 @@ def measure_small_launches(shapes=SMALL_LAUNCH_SHAPES, *, bn=256, bk=512, seed=0
     """Strassen and the cubic on operands packed once (outside the timing),
     no epilogue, against hipBLASLt, on launches whose few tiles leave most
     CUs idle unless the K split spreads them; the arms rotate per sample of
-    ``batch`` back-to-back calls. The split's share count comes from the
-    library (``smx_gemm_workspace_bytes``); run once as is and once with
-    SMX_TAIL_SPLIT=0 to time the whole tiles."""
+    ``batch`` back-to-back calls. The Strassen call's share count comes from
+    the library (``smx_matmul_plan``); run once as is and once with
+    SMX_TAIL_SPLIT=0 to time K undivided."""
     emit = emit or (lambda record: None)
     device = torch.device(device)
     cus = torch.cuda.get_device_properties(device).multi_processor_count

@@ -134,6 +134,15 @@ for algo in (7, 8):
     subprocess.run([sys.executable, "-c", script], env=env, check=True)
 
 
+@pytest.mark.parametrize("algo", [7, 8])
+def test_recorded_shares_are_those_of_the_call(algo):
+    """On the streaming kernel too, whose shares differ from smx_gemm's (12 here)."""
+    for m, k, n in ((16, 25600, 5120), (256, 25600, 5120), (8192, 5120, 5120)):
+        bm = min(m, 256)
+        assert _lib.k_shares(m, k, n, (bm, 256, 512), algo, CUS) == plan(m, k, n, algo=algo, bm=bm).shares
+    assert _lib.k_shares(16, 25600, 5120, (16, 256, 512), algo, CUS) == 6
+
+
 def test_plan_checks_its_arguments():
     lib, d = _lib.load(), _lib.SmxGemmDesc()
     p = _lib.SmxMatmulLaunch()

@@ -308,8 +308,8 @@ struct Params {
   int32_t ksplit;
   int32_t tile_base;
   int64_t split_stride;
-  // Product-major Strassen kernel (kernel_pm.hpp): FP32 space for one parked
-  // quadrant set per workgroup (pm::kParkBytes each). Streaming kernel
+  // Product-major Strassen kernel (kernel_pm.hpp): FP32 space for two parked
+  // partial sets per workgroup (pm::kParkBytes for both). Streaming kernel
   // (kernel_stream.hpp): the FP32 [m, n] shares of a K-divided launch.
   void* park;
   int32_t epilogue;  // SMX_EPI_* of a kernel that chooses it at run time

@@ -350,21 +350,6 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_packed(Params p) {
 
 }
 
-// Packs one operand stored with its rows contiguous, [k, rows], whatever its
-// alignment (pack_rows and pack_cols below take the others). kSide 0: A
-// [m, k] (stored [k, m]), product row R = (tile i,
-// row r < bm/2) -> physical rows i*bm + r (top) and + bm/2 (bottom).
-// kSide 1: B^T [n, k] (stored [k, n]), product column C = (tile j, c < bn/2) ->
-// rows j*bn + c (left) and + bn/2 (right) of B^T. Product depth k' = (panel
-// s, kk < bk/2) -> columns s*bk + kk and + bk/2. Quadrants: A0 = (top, k
-// left), A1 = (top, k right), A2 = (bottom, k left), A3 = (bottom, k right);
-// B0 = (k top, left), B1 = (k top, right), B2 = (k bottom, left),
-// B3 = (k bottom, right) (strassen_pallas.py:188-204). With a panel map,
-// packed K panel s reads source panel panels[s] (the Strassen or the exact
-// panels of an exact-panel schedule); without one, panel s. One wave packs one
-// 32-row product block over kPackStages stages: each lane gathers eight
-// elements of each quadrant per stage and stores nops 16-byte chunks, so the stores of
-// a wave are whole 1 KB fragments.
 // One lane's share of one packed stage: from the four quadrant values x
 // (A: [row half][K half]; B: [K half][column half]) of its 8 consecutive k,
 // the nops operands of the formula, each stored as 16 bytes at dst + op x 4 KB
@@ -391,6 +376,21 @@ __device__ __forceinline__ void store_fragments(F8 (&x)[4], int formula, int per
   }
 }
 
+// Packs one operand stored with its rows contiguous, [k, rows], whatever its
+// alignment (pack_rows and pack_cols below take the others). kSide 0: A
+// [m, k] (stored [k, m]), product row R = (tile i,
+// row r < bm/2) -> physical rows i*bm + r (top) and + bm/2 (bottom).
+// kSide 1: B^T [n, k] (stored [k, n]), product column C = (tile j, c < bn/2) ->
+// rows j*bn + c (left) and + bn/2 (right) of B^T. Product depth k' = (panel
+// s, kk < bk/2) -> columns s*bk + kk and + bk/2. Quadrants: A0 = (top, k
+// left), A1 = (top, k right), A2 = (bottom, k left), A3 = (bottom, k right);
+// B0 = (k top, left), B1 = (k top, right), B2 = (k bottom, left),
+// B3 = (k bottom, right) (strassen_pallas.py:188-204). With a panel map,
+// packed K panel s reads source panel panels[s] (the Strassen or the exact
+// panels of an exact-panel schedule); without one, panel s. One wave packs one
+// 32-row product block over kPackStages stages: each lane gathers eight
+// elements of each quadrant per stage and stores nops 16-byte chunks, so the
+// stores of a wave are whole 1 KB fragments.
 template <int kAlgo, int kSide, bool kF32>
 __global__ __launch_bounds__(256) void pack_operand(const void* __restrict__ src_v, int64_t ld, int64_t rows,
                                                     int64_t k, int32_t tile_rows, int32_t bk, int32_t formula,

@@ -4,11 +4,12 @@
 //
 // Why: gemm_split keeps the seven products of a 128 x 128 product tile in
 // registers for the whole K loop (448 registers per lane), so each 1 KB
-// operand fragment it streams from L2 into LDS feeds four MFMAs: 512 bytes
-// per MFMA, twice the matched cubic's, which keeps the texture address unit
-// (TA, 16 cycles per 64-lane 16-byte DMA) as busy as the MFMAs. Three sets
-// of a 128 x 256 tile are 384 registers per lane, and each A fragment feeds
-// 4 MFMAs, each B fragment 2: 384 bytes per MFMA.
+// operand fragment it streams from L2 into LDS feeds four MFMAs (of 32 x 32 x
+// 16): 512 bytes per MFMA, twice the matched cubic's, which keeps the texture
+// address unit (TA, 16 cycles per 64-lane 16-byte load) as busy as the MFMAs.
+// Three sets of a 128 x 256 tile are 384 registers per lane; each fragment of
+// the tile's four row blocks meets eight column blocks and the other way
+// round, 384 bytes for the same work.
 //
 // The products contribute to the four output quadrants as
 //   C0 = P1 + P4 - P5 + P7,  C1 = P3 + P5,  C2 = P2 + P4,  C3 = P1 - P2 + P3 + P6
@@ -38,13 +39,17 @@
 //
 // Waves: wave w owns all 128 product rows and columns 64 w .. + 63 of the
 // tile, 8 x 4 blocks of 16 x 16 per set; per 32 k it uses 8 A and 4 B
-// fragments for 32 MFMAs of 16 x 16 x 32. A's fragments are shared by the four waves and go
-// through LDS; B's belong to one wave each and go straight into its
+// fragments (16 x 32) for 32 MFMAs of 16 x 16 x 32, so an A fragment feeds 4 of
+// its MFMAs and a B fragment 8. A's fragments are shared by the four waves and
+// go through LDS; B's belong to one wave each and go straight into its
 // registers. LDS then carries 64 KB of reads and 16 KB of DMA writes per
 // 1024 cycles of MFMAs; with both operands in LDS and 64 x 128 waves it was
 // 96 and 48 KB, more than its 128 bytes a cycle. Gate|up call (8192 x 5120 x
 // 51200, SwiGLU): 3.488 -> 3.364 ms; with the stage addresses kept
-// incrementally (Stream) and one wait per half step 3.30, power limited.
+// incrementally (Stream) and one wait per half step 3.30. What bounds it now is
+// the operand path: on that call's head the data return unit (TD) is busy or
+// waiting 98% of the cycles, half of them stalled on the L1, the MFMA pipe busy
+// 61% (the cubic 70% and 69%), at a clock of about 1.8 of 2.4 GHz.
 //
 // Pipeline: a stage is kQ 16-k steps of one product. B is loaded one stage
 // ahead (kQ = 8: 2048 cycles of MFMAs), A's ring is refilled kSlots - 1

@@ -31,15 +31,18 @@
 //      tiles, 64x64 waves, both operands pre-packed (smx_pack_operand: the
 //      Strassen operand sums or the cubic quadrants, in MFMA fragment order)
 //      and streamed into an LDS ring by DMA.
+//   pm (kernel_pm.hpp): Strassen on whole rounds of 128x256 tiles, the seven
+//      products one after another into three accumulator sets.
 //   stream (kernel_stream.hpp): launches of few product rows or few tiles
-//      (smx_matmul): tiles of 32 to 128 rows and columns, one product per wave,
-//      operands straight from memory into registers.
+//      (smx_matmul): tiles of 32 or 64 product rows and 32 to 128 columns, one
+//      Strassen product (two of the cubic's) per wave, operands straight from
+//      memory into registers.
 //   v1 (kernel_v1.hpp): 128x64 tiles, row-major A and B^T, both operand sums
 //      formed in registers; serves unpacked calls whose tile the packed
 //      kernels cannot take, or all of them under SMX_PLAIN_WEIGHTS=compact.
-// The split and packed kernels are instantiated in translation units of
-// their own (gemm_strassen*.hip, gemm_cubic*.hip) and reached through the
-// launchers of launch.hpp; a thin tiling (bm/2 not a multiple of the 128-row
+// All but v1 are instantiated in translation units of their own
+// (gemm_strassen*.hip, gemm_cubic*.hip, gemm_stream.hip) and reached through
+// the launchers of launch.hpp; a thin tiling (bm/2 not a multiple of the 128-row
 // product tile, bm % 16 == 0 as the reference allows) runs their kThin
 // instantiations, whose epilogues map rows one by one (ThinRows).
 
